@@ -313,8 +313,8 @@ DEV T sel_of(const T (&v)[N], int idx) {
 // number of rounds that all waves agree on, so that every barrier is reached by all.
 //
 // FX = 1 builds the kernel for the common configuration (PF, chase combining, EESM, RLC AM, OLLA, PHR cap, retx
-// priority, a fixed Rician phasor, fading; fx_profile), FX = 2 for the same without the Rician phasor: those
-// switches become compile-time constants, which removes their tests from the slot loop and the scalar registers that
+// priority, fading, with a fixed Rician phasor or without: then its K and phasor are 0, and the gain's 0 0 + 1 h is h
+// bit for bit; fx_profile), FX = 2 for the same without the Rician phasor: those switches become compile-time constants, which removes their tests from the slot loop and the scalar registers that
 // hold them.
 // Minimum waves per SIMD (the register budget): 2, and 3 for the two-wave FX = 2 build (envs of 65..128 robots at the
 // common configuration: 168 VGPRs with 104 B per lane of spills, measured 7% faster than 193 VGPRs at 2 waves on
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     INET_PH_DECL
     InetNrParams pm = pm_in;
     InetNrTables tb = tb_in;
-    if constexpr (FX == 1 || FX == 2) {
+    if constexpr (FX != 0) {
         pm.sched = 0; pm.comb = 1; pm.eesm = 1; pm.harq_drop = 0; pm.olla = 1; pm.phr_cap = 1; pm.retx_prio = 1;
         pm.rician = FX == 1 ? 1 : 0; pm.fading = 1;
         pm.pf_rbg = 0; pm.pf_freeze = 0; pm.whole_band = 0; pm.pc1_on = 0; pm.retx_tdma = 0; pm.amc_prev = 0;
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         sp_re[c] = 0.f; sp_im[c] = 0.f; kk[c] = 0.f; kf[c] = 0.f; kg[c] = 0;
-        if (pm.rician && act) {
+        if (pm_in.rician && pm.rician && act) {
             sp_re[c] = ldo(st.spec_re, o_rc(c)); sp_im[c] = ldo(st.spec_im, o_rc(c)); kk[c] = ldo(st.k_lin, o_rc(c));
         }
     }
@@ -2343,7 +2343,7 @@ void launch_step(const StepArgs& a) {
                            a.n_data, a.arr, none);
 }
 
-// the build that fixes these parameters at compile time: 1 (with the Rician phasor) or 2 (without), 0 for none
+// the build that fixes these parameters at compile time: 2 (no Rician phasor), 1 (a fixed Rician K), 0 for none
 inline int fx_profile(const InetNrParams& p) {
     const bool common = p.pf_rbg == 0 && p.pf_freeze == 0 && p.whole_band == 0 && p.pc1_on == 0 &&
                         p.retx_tdma == 0 && p.amc_prev == 0 && p.fc_on == 0 && p.los_sto == 0 && p.k_from_los == 0 &&
@@ -2378,12 +2378,21 @@ void launch_step_mc(const StepArgs& a) {
                        a.arr, *a.cells);
 }
 
-// every (P, IR, per-subband SNR) with a runtime segment width; plus, for 32-robot envs without IR or per-subband
-// input, a build with the width fixed at compile time
+// every (P, IR, per-subband SNR) with a runtime segment width; plus, for segments of 32 lanes without IR or per-subband
+// input, a build with the width fixed at compile time, and the common configuration's builds
 template <int S>
 StepFn pick_step_s(int P, bool ir, bool vref, int rb, int fx) {
-    if constexpr (S == 13)                           // the common configuration at 13 RBGs, 8 HARQ, 32-robot envs
-        if (fx == 1 && P == 8 && !ir && !vref && rb == 32) return &launch_step<13, 8, false, false, 32, 1>;
+    // the common configuration (with or without the Rician phasor) at 8 or 16 HARQ processes in segments of 32 or 64
+    // lanes. The general build keeps every switch's branch and scalar registers live and spills 264..456 B per lane to
+    // scratch at these process counts; against it at the same width (13 RBGs): 16 processes, 256 x 16 in 64 lanes,
+    // 20 UL slots, 612 -> 495 us; 1024 x 32 in 64 lanes, 8 UL slots, 328 -> 264 us, in 32 lanes 412 -> 364 us;
+    // 8 processes, 1024 x 32 in 64 lanes, 10 UL slots, 198 -> 154 us.
+    if (fx != 0 && !ir && !vref) {
+        if (P == 8 && rb == 32) return &launch_step<S, 8, false, false, 32, 1>;
+        if (P == 8 && rb == 64) return &launch_step<S, 8, false, false, 64, 1>;
+        if (P == 16 && rb == 32) return &launch_step<S, 16, false, false, 32, 1>;
+        if (P == 16 && rb == 64) return &launch_step<S, 16, false, false, 64, 1>;
+    }
 #define INET_PICK(PP)                                                                                 \
     if (P == PP) {                                                                                    \
         if (!ir && !vref && rb == 32) return &launch_step<S, PP, false, false, 32>;                  \
@@ -2432,6 +2441,10 @@ template <int S>
 StepFn pick_step_w2_s(int P, bool ir, int fx) {
     if constexpr (S == 8)                            // config 5's switches without the Rician phasor, 8 HARQ
         if (fx == 2 && P == 8 && !ir) return &launch_step_w2<8, 8, false, 2>;
+    // the common configuration (13 RBGs, 16 processes, 4096 x 100, 8 UL slots: 1863 us in the general build, with 392 B
+    // per lane of scratch, 1593 us in this one)
+    if (fx != 0 && P == 8 && !ir) return &launch_step_w2<S, 8, false, 1>;
+    if (fx != 0 && P == 16 && !ir) return &launch_step_w2<S, 16, false, 1>;
 #define INET_PICK_W2(PP) \
     if (P == PP) return ir ? &launch_step_w2<S, PP, true> : &launch_step_w2<S, PP, false>;
     INET_PICK_W2(2) INET_PICK_W2(4) INET_PICK_W2(8) INET_PICK_W2(16)
