@@ -109,7 +109,7 @@ class HipWifiEngine:
             raise HipUnsupported(f"hidden nodes with R + A = {R + self.A}: (R + A)^2 < 400, the size up to which the "
                                  "reference's sensing-matrix products add in index order")
         rb = 1 << max(0, (R - 1).bit_length())
-        self.envs_per_wave = int(envs_per_wave) if envs_per_wave is not None else 1
+        self.envs_per_wave = int(envs_per_wave) if envs_per_wave is not None else self._auto_envs_per_wave(rb)
         if self.envs_per_wave < 1 or self.envs_per_wave * rb > 64:
             raise ValueError(f"envs_per_wave must be in 1..{64 // rb} for R={R}")
         self._alloc_state()
@@ -117,6 +117,21 @@ class HipWifiEngine:
         self.reset(None)
 
     # ------------------------------------------------------------------ buffers and constants
+    # wavefronts of a step that the chip holds at once: the mean-field kernel takes one per SIMD (its registers), so one
+    # more starts a second round of the whole serial chain; the per-slot kernel two or more. us per step by envs per
+    # wavefront, mean-field 2048 x 16: 437 (one), 230 (two); 4096 x 6: 1138, 583, 302, 306 (1, 2, 4, 8); 1024 x 16: 223,
+    # 231; per-slot 4096 x 16: 94, 68, 73 (1, 2, 4), 2048 x 30: 70, 73 (1, 2)
+    _waves = 1024
+
+    def _auto_envs_per_wave(self, rb):
+        """The launch's envs per wavefront, in segments of rb = next_pow2(R) lanes (mean-field: of next_pow2(R + A)):
+        the fewest with which every wavefront of the batch is resident, or all that fit."""
+        seg = rb if self.level == "WIFI_DCF" else min(64, 1 << (self.R + self.A - 1).bit_length())
+        g = 1
+        while 2 * g * seg <= 64 and -(-self.E // g) > self._waves:
+            g *= 2
+        return 1 if g == 1 else min(64 // rb, g * seg // rb)
+
     def _alloc_state(self):
         E, R, F, d = self.E, self.R, self.F, self.dev
         i32, f32 = torch.int32, torch.float32
@@ -569,6 +584,7 @@ class HipWifiDcfEngine(HipWifiEngine):
     stated in full in include/inet_wifi.h and oracle/dcf_oracle.py's module docstring."""
 
     level = "WIFI_DCF"
+    _waves = 2048
 
     def __init__(self, E, R, device="cuda", cfg: NRConfig | None = None, seed=None, envs_per_wave=None):
         cfg = cfg if cfg is not None else NRConfig()
