@@ -303,6 +303,27 @@ bool rlf_ok(const InetNrCells& c, bool step) {
 
 int next_pow2(int v) { int p = 1; while (p < v) p <<= 1; return p; }
 
+// The lanes of a wavefront that one env of next_pow2(R) = rb0 lanes takes: rb0, or twice, four times, ... that while the
+// batch still leaves the chip room. A wavefront's time is its serial chain of slots, and the work that its envs deal
+// over the 64 lanes (fading draws, estimates, the MCS search) grows with the envs it holds, so a batch that does not
+// fill the chip is spread over more wavefronts with fewer envs each, down to one env per wavefront. The room is one
+// wavefront for each of the 1024 SIMDs, or the `occ` that are resident on one; past one per SIMD an env takes at most
+// four times its own lanes, and the DL launch, whose short slots gain nothing, keeps to one per SIMD. Measured, us per
+// step in 8 / 16 / 32 / 64 lanes per env: 64 x 8 round robin 99.9 / 88.8 / 80.4 / 81.2, 2048 x 8 104 / 96 / 89 / 103;
+// default configuration 256 x 16 (20 UL slots) - / 1202 / 679 / 495, 2048 x 16 (8 UL slots) - / 579 / 328 / 276,
+// 4096 x 16 - / 573 / 371 / 511, 1024 x 32 - / - / 364 / 264, 4096 x 32 - / - / 443 / 575; UL and DL 2048 x 32
+// - / - / 524 / 544; three cells (one wavefront per SIMD) 1024 x 16 - / 728 / 552 / 354, 2048 x 32 - / - / 813 / 894.
+int seg_width(int E, int rb0, int occ, bool dl) {
+    constexpr int64_t SIMDS = 1024;
+    int rb = rb0;
+    while (rb < inet::STEP_WAVE) {
+        const int64_t waves = ((int64_t)E * 2 * rb + inet::STEP_WAVE - 1) / inet::STEP_WAVE;
+        if (waves > SIMDS && (dl || 2 * rb > 4 * rb0 || waves > occ * SIMDS)) break;
+        rb *= 2;
+    }
+    return rb;
+}
+
 // the argument checks and the launch of one step kernel (UL: dl NULL)
 int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const InetNrTables* tab,
                            const InetNrParams* prm, const InetNrRow* rows, int32_t n_rows, int64_t T, const float* x,
@@ -331,7 +352,7 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
         return INET_NR_EINVAL;
     const int n_data = p.n_data > 0 ? p.n_data : n_rows;
     const bool ir = p.comb == 2, vref = p.input_kind == 2;
-    const int rb = next_pow2(p.R);
+    const int rb = seg_width(p.E, next_pow2(p.R), cells ? 1 : 2, dl != nullptr);
     // the single-cell entry points run one cell; inet_nr_step_cells several
     if ((cells != nullptr) != (p.n_cells > 1)) return INET_NR_EINVAL;
     inet::StepFn fn;
