@@ -299,6 +299,37 @@ DEV T sel_of(const T (&v)[N], int idx) {
     return r;
 }
 
+// The step kernel's arguments, one struct at the start of the kernel argument segment. lk is the DL link's state (the UL
+// build reads st; its lk holds nothing).
+struct NoLink {};
+template <class LS>
+struct StepKernArgs {
+    InetNrState st;
+    std::conditional_t<std::is_same<LS, InetNrState>::value, NoLink, LS> lk;
+    InetNrTables tb;
+    InetNrParams pm;
+    const InetNrRow* rows;
+    int64_t T;
+    const float* x;
+    const int64_t* hid;
+    int n_rows, rb, n_ul_max;
+    InetNrOutputs out;
+    InetNrArrivals arr;
+    InetNrCells cl;
+};
+// The kernel's arguments read again from here on: the empty asm hides that the address is the one the kernel began
+// with, so the fields come from the scalar cache where they are used instead of being held in scalar registers since
+// the kernel's start: they do not fit, and a spilled one costs a lane read and a hazard wait at each use. Read again for the end of
+// the step and in every slot, the common build at 13 RBGs spills 86 scalars instead of 233: rl 4096 x 32 216.4 -> 211.2
+// us, 3000 x 20 at 14 RBGs 171.0 -> 161.5, 16384 x 128 2625 -> 2574.
+template <class LS>
+DEV const StepKernArgs<LS>& args_again() {
+    const __attribute__((address_space(4))) char* p =
+        (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const StepKernArgs<LS>*)p;
+}
+
 // RBT: the segment width when it is fixed at compile time (0: the runtime argument rb).
 // LS: the link whose MAC state and queue the kernel runs: InetNrState (the UL; lk is st) or InetNrDlState (the DL
 // of NRConfig(dl=True): CQI reports and DL data slots with the DlMac hooks; it reads the shared state of st and writes
@@ -322,12 +353,19 @@ DEV T sel_of(const T (&v)[N], int idx) {
 template <int S, int P, bool IR, bool VREF, int RBT, class LS, int NC, int FX = 0>
 __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1),
                              NC > 1 ? 1 : ((RBT == 128 && FX == 2) ? 3 : 2)) void nr_step_kernel(
-    InetNrState st, LS lk_in, InetNrTables tb_in, InetNrParams pm_in, const InetNrRow* __restrict__ rows, int n_rows,
-    int64_t T_arg, const float* __restrict__ xin, const int64_t* __restrict__ cur_hid, InetNrOutputs out, int rb_arg,
-    int n_ul_max, InetNrArrivals arr, InetNrCells cl) {
+    const StepKernArgs<LS> args) {
+    const InetNrState& st = args.st;
+    const InetNrParams& pm_in = args.pm;
+    const InetNrRow* const __restrict__ rows = args.rows;
+    const float* const __restrict__ xin = args.x;
+    const int64_t* const __restrict__ cur_hid = args.hid;
+    const int n_rows = args.n_rows, n_ul_max = args.n_ul_max;
+    const InetNrOutputs& out = args.out;
+    const InetNrArrivals& arr = args.arr;
+    const InetNrCells& cl = args.cl;
     INET_PH_DECL
     InetNrParams pm = pm_in;
-    InetNrTables tb = tb_in;
+    const InetNrTables& tb = args.tb;
     if constexpr (FX != 0) {
         pm.sched = 0; pm.comb = 1; pm.eesm = 1; pm.harq_drop = 0; pm.olla = 1; pm.phr_cap = 1; pm.retx_prio = 1;
         pm.rician = FX == 1 ? 1 : 0; pm.fading = 1;
@@ -336,7 +374,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     }
     constexpr bool DL = !std::is_same<LS, InetNrState>::value;
     // the link whose MAC state the kernel runs: the UL link is the shared state itself (one set of pointers)
-    const LS& lk = [&]() -> const LS& { if constexpr (DL) return lk_in; else return st; }();
+    const LS& lk = [&]() -> const LS& { if constexpr (DL) return args.lk; else return args.st; }();
     constexpr bool MC = NC > 1;
     static_assert(!(MC && (DL || VREF)), "several cells: the UL with pose input");
     constexpr int W = RBT > STEP_WAVE ? RBT / STEP_WAVE : 1;   // wavefronts per env (1, 2 or 4)
@@ -344,8 +382,8 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     constexpr int CW = STEP_WAVE * W;                   // lanes per workgroup (the LDS column stride)
     static_assert(!(MC && W > 1), "several cells: one wavefront per env");
     constexpr int NCS = NC * S;                        // fading links per robot (cell-major, subband-minor)
-    const int rb = RBT ? RBT : rb_arg;
-    const int64_t T = T_arg >= 0 ? T_arg : st.clock[0];
+    const int rb = RBT ? RBT : args.rb;
+    const int64_t T = args.T >= 0 ? args.T : st.clock[0];
     extern __shared__ int dyn[];
     __shared__ __align__(16) float s_thr[MAX_M];
     __shared__ __align__(16) float s_thrs[MAX_M];                // suffix minima of s_thr (the MCS search table)
@@ -981,7 +1019,11 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     INET_PH(0);                                    // prologue: tables, state loads, arrivals, radio
     // ================================================================ slot loop
     for (int k = 0; k < n_rows; ++k) {
-        const InetNrRow row = rows[k];
+        // (the slot's constants and table pointers come from the scalar cache in every slot)
+        const StepKernArgs<LS>& args = args_again<LS>();
+        const InetNrParams& pv = args.pm;
+        const InetNrTables& tb = args.tb;
+        const InetNrRow row = args.rows[k];
         const int g = g0 + row.rel;
         if (k_ramps) {
 #pragma unroll
@@ -1197,14 +1239,14 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 ni_la[s] = 10.0f * log10f(s_ni[serv * S + s]);
-                ref[s] = (pm.ref_off + pg_s) - ni_la[s];
+                ref[s] = (pv.ref_off + pg_s) - ni_la[s];
             }
-            const float rx_s = pg_s + pm.ue_tx;
-            if (cl.pc_on) pc = pm.ue_tx - (cl.pc_p0 + cl.pc_alpha * (pm.ue_tx - rx_s));
+            const float rx_s = pg_s + pv.ue_tx;
+            if (cl.pc_on) pc = pv.ue_tx - (cl.pc_p0 + cl.pc_alpha * (pv.ue_tx - rx_s));
             n_max = S;
             if (pm.phr_cap && !pm.whole_band) {
-                const float phr = rx_s - pm.subband_noise;
-                float f = floorf((pm.snr_ref_prbs * from_db(phr - pm.phr_min)) / pm.w0);
+                const float phr = rx_s - pv.subband_noise;
+                float f = floorf((pv.snr_ref_prbs * from_db(phr - pv.phr_min)) / pv.w0);
                 n_max = (int)clampf(f, 1.0f, (float)S);
             }
             unsigned long long cm[NC];
@@ -1261,7 +1303,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         } else {
             // grants (UlMac._pre_slot_lumped)
             if (row.flags & 16) bsr = bsr > 1 ? bsr : 1;
-            if (sr_t >= 0 && g - sr_t >= pm.sr_delay) { bsr = bsr > 1 ? bsr : 1; sr_t = -1; }
+            if (sr_t >= 0 && g - sr_t >= pv.sr_delay) { bsr = bsr > 1 ? bsr : 1; sr_t = -1; }
         }
         // candidates: the retransmission ready first (lowest ready slot, then lowest process), the lowest free process
         int rx_p = 0, p_new = 0;
@@ -1303,7 +1345,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     // UL: the PSD over one RBG, at most the power-control PSD (mac_ul.py:154-171); DL: sinr_ref + csi
                     // (mac_dl.py:42-43)
                     // (ul_power "whole_band": the fixed PSD over the carrier, mac_ul.py:157-160)
-                    const float wdb = pm.whole_band ? pm.wb_db : s_wdb[s];
+                    const float wdb = pm.whole_band ? pv.wb_db : s_wdb[s];
                     const float wd = use_pc ? (wdb > pc ? wdb : pc) : wdb;
                     const float est = DL ? REF(s) + csi[s] : (REF(s) - wd) + csi[s];
                     s_eo[s * CW + lane] = pm.olla ? est + olla : est;
@@ -1517,9 +1559,9 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         uint32_t won = 0;
         // pf_update "rbg" (mac.py:325-329, 526-532): the metric of RBG s is rate_s / max(base + wwin got, 1e-9) with
         // base = (1 - wwin) avg and got the rate of the RBGs this robot won so far in the slot
-        const float pf_base = pm.pf_a * avg;
+        const float pf_base = pv.pf_a * avg;
         float got = 0.f;
-        auto rbg_metric = [&](int s) { return DivBy(clamp_min(pf_base + pm.pf_b * got, 1e-9f))(rate[s]); };
+        auto rbg_metric = [&](int s) { return DivBy(clamp_min(pf_base + pv.pf_b * got, 1e-9f))(rate[s]); };
         // (one copy of the loop per retx-priority setting, so that the test is not repeated per RBG)
         auto allocate = [&](auto retx_prio) {
             constexpr bool RP = decltype(retx_prio)::value;
@@ -1568,7 +1610,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         const bool tx_new = new_el && n_sb > 0;
         const bool tx = tx_rx || tx_new;
         // power split (mac_ul.py:173-180): PUSCH power spread over n_prb PRBs, at least the power-control backoff
-        const float sp0 = pm.whole_band ? pm.wb_db : 10.0f * log10_clamped(clamp_min(n_prb / pm.snr_ref_prbs, 1e-3f));
+        const float sp0 = pm.whole_band ? pv.wb_db : 10.0f * log10_clamped(clamp_min(n_prb / pv.snr_ref_prbs, 1e-3f));
         const float sp = use_pc ? (sp0 > pc ? sp0 : pc) : sp0;
         // log of the held PRB count as torch computes it: logsumexp of log w over the held RBGs
         const float lnw = lw_eq ? s_lnw[__popc(won)] : lse_logw<S>(s_logw, won);
@@ -1729,7 +1771,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     if (tbs_m > 0) {
                         float b = bler_at(tb.bler, (m * tb.C + ci0) * tb.G, tb.G, tb.s0, tb.ds, rds, eff, cwi);
                         float tbler = 1.0f - pow_count(1.0f - b, ncb);
-                        pass = tbler <= pm.target;
+                        pass = tbler <= pv.target;
                     }
                 }
                 const unsigned long long pb = __ballot(pass);
@@ -1751,7 +1793,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             }
         }
         INET_PH(5);                                // link adaptation (power split, lse of log w, MCS search)
-        int cap_b = tbs_new / 8 - pm.tb_oh;
+        int cap_b = tbs_new / 8 - pv.tb_oh;
         cap_b = cap_b > 1 ? cap_b : 1;
         const int byt_new = cap_b < unsent ? cap_b : unsent;
         // ---- bind TBs to HARQ processes (mac.py:407-426) ----
@@ -1802,7 +1844,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     // the robot's PSD at every cell: ((pg_c + ue_tx) - ref_db) - split
                     float* const s_psd = s_ipsd;
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) s_psd[c * STEP_WAVE + lane] = ((pgc[c] + pm.ue_tx) - cl.ref_db) - sp;
+                    for (int c = 0; c < NC; ++c) s_psd[c * STEP_WAVE + lane] = ((pgc[c] + pv.ue_tx) - cl.ref_db) - sp;
 #pragma unroll
                     for (int s = 0; s < S; ++s) {
                         if (txing && ((won >> s) & 1u)) {
@@ -1835,7 +1877,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                 } else {                                // several envs per wavefront: each lane its own terms
 #pragma unroll
                     for (int c = 0; c < NC; ++c) {
-                        const float psd = ((pgc[c] + pm.ue_tx) - cl.ref_db) - sp;
+                        const float psd = ((pgc[c] + pv.ue_tx) - cl.ref_db) - sp;
 #pragma unroll
                         for (int s = 0; s < S; ++s) {
                             float v = 0.f;
@@ -1917,12 +1959,12 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             float u = uniform_bits(elem_hash(mix32(base0 ^ row.salt_bler), (uint32_t)r));
             ok = tx && u >= p_err;
             fail = tx && !ok;
-            exh = fail && ntx >= pm.max_tx;
+            exh = fail && ntx >= pv.max_tx;
         }
         INET_PH(7);                                // decoding
         // ---- HARQ state update (mac.py:456-477; UL timing mac_ul.py:218-219, DL mac_dl.py:47-49: decoded TBs wait
         // for their HARQ-ACK at the row's ACK slot, and both outcomes are known gnb_proc slots after it) ----
-        int rdy_ok = g, rdy_fail = g + pm.ul_rtt, st_ok = 0;
+        int rdy_ok = g, rdy_fail = g + pv.ul_rtt, st_ok = 0;
         if constexpr (DL) {
             rdy_ok = g0 + ((row.flags >> 8) & 0xffff) + lk.gnb_proc;
             rdy_fail = rdy_ok;
@@ -1942,14 +1984,14 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     else {
                         ntxp = 0; hcomb[p] = 0.f;
                         if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
-                        hrdy[p] = g + pm.rlc_retx;
+                        hrdy[p] = g + pv.rlc_retx;
                     }
                 }
                 hmeta[p] = hm_pack(stp, ntxp, hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
             }
         }
         // ---- OLLA, BSR, PF average, RR (mac.py:479-485, mac_ul.py:229-236, mac.py:534-554) ----
-        if (pm.olla) olla = clampf((olla + pm.olla_up * (ok ? 1.0f : 0.0f)) - pm.olla_dn * (fail ? 1.0f : 0.0f),
+        if (pm.olla) olla = clampf((olla + pv.olla_up * (ok ? 1.0f : 0.0f)) - pv.olla_dn * (fail ? 1.0f : 0.0f),
                                    -10.0f, 10.0f);
         const int served = ok ? hi_tx - lo_tx : 0;
         if (!DL && tx) bsr = enq - sent;
@@ -1958,7 +2000,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             // PF average (mac.py:534-554): EWMA of the served bytes; pf_update "rbg": of the granted bytes of a new TB;
             // pf_avg_idle "freeze": only robots with new data to schedule in this slot move it
             const float upd = pm.pf_rbg ? (float)(tx_new ? tbs_new / 8 : 0) : (float)served;
-            const float na = clamp_min(pm.pf_a * avg + pm.pf_b * upd, 1e-9f);
+            const float na = clamp_min(pv.pf_a * avg + pv.pf_b * upd, 1e-9f);
             avg = (pm.pf_freeze && !(need > 0 && !has_rx)) ? avg : na;
         }
         if (pm.sched == 2 && tx) last_tx = g;
@@ -1968,7 +2010,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         c_prb += tx ? (int)n_prb : 0;
         if (lena) { c_tbb += tx_new ? tbs_new / 8 : 0; c_tbe += (tx_new && byt_new == 0) ? 1 : 0; }
         if (tx) {
-            int kh = ntx < pm.max_tx ? ntx : pm.max_tx;
+            int kh = ntx < pv.max_tx ? ntx : pv.max_tx;
             atomicAdd(&my_hist[HB + kh], 1);
             atomicAdd(&my_hist[(ok ? 0 : 2 * HB) + kh], 1);
         }
@@ -2011,6 +2053,14 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     const int n_hist = DL ? 0 : (n_ul < n_ul_max ? n_ul : n_ul_max);
 
     // ================================================================ end of step (NRNet._finish)
+    {
+    const StepKernArgs<LS>& args = args_again<LS>();
+    const InetNrState& st = args.st;
+    const LS& lk = [&]() -> const LS& { if constexpr (DL) return args.lk; else return args.st; }();
+    const InetNrOutputs& out = args.out;
+    const InetNrArrivals& arr = args.arr;
+    const InetNrCells& cl = args.cl;
+    const int64_t* const __restrict__ cur_hid = args.hid;
     if constexpr (MC) {                            // A3 triggers after the step's last active slot (nr_engine.py:780)
         const bool late = cl.rlf ? rlf_events(g0 + N - 1) : (act && !fired && k_ho >= 0);
         if (late) handover(g0 + k_ho);
@@ -2305,6 +2355,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         if (r == 0)
             for (int q = rb; q < 3 * HB; ++q) lk.hist[(size_t)e * 3 * HB + q] += my_hist[q];
     }
+    }
     INET_PH(11);                                      // state stores, per-env reductions and counters
     INET_PH_STORE;
 }
@@ -2330,17 +2381,26 @@ struct StepArgs {
 };
 typedef void (*StepFn)(const StepArgs&);
 
+template <class LS>
+StepKernArgs<LS> kern_args(const StepArgs& a) {
+    StepKernArgs<LS> k{};
+    k.st = a.st;
+    if constexpr (!std::is_same<LS, InetNrState>::value) k.lk = *a.dl;
+    k.tb = a.tb; k.pm = a.pm; k.rows = a.rows; k.T = a.T; k.x = a.x; k.hid = a.hid;
+    k.n_rows = a.n_rows; k.rb = a.rb; k.n_ul_max = a.n_data;
+    k.out = a.out; k.arr = a.arr;
+    if (a.cells) k.cl = *a.cells;
+    return k;
+}
+
 template <int S, int P, bool IR, bool VREF, int RBT, int FX = 0>
 void launch_step(const StepArgs& a) {
-    const InetNrCells none{};
     if (a.dl)
         hipLaunchKernelGGL((nr_step_kernel<S, P, IR, VREF, RBT, InetNrDlState, 1, FX>), dim3(a.grid),
-                           dim3(STEP_WAVE), a.lds, a.stream, a.st, *a.dl, a.tb, a.pm, a.rows, a.n_rows, a.T, a.x,
-                           a.hid, a.out, a.rb, a.n_data, a.arr, none);
+                           dim3(STEP_WAVE), a.lds, a.stream, kern_args<InetNrDlState>(a));
     else
         hipLaunchKernelGGL((nr_step_kernel<S, P, IR, VREF, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(STEP_WAVE),
-                           a.lds, a.stream, a.st, a.st, a.tb, a.pm, a.rows, a.n_rows, a.T, a.x, a.hid, a.out, a.rb,
-                           a.n_data, a.arr, none);
+                           a.lds, a.stream, kern_args<InetNrState>(a));
 }
 
 // the build that fixes these parameters at compile time: 2 (no Rician phasor), 1 (a fixed Rician K), 0 for none
@@ -2357,25 +2417,21 @@ inline int fx_profile(const InetNrParams& p) {
 // or SNR input; the UL, and with RBT = 128 the DL too)
 template <int S, int P, bool IR, int FX = 0, int RBT = 128>
 void launch_step_w2(const StepArgs& a) {
-    const InetNrCells none{};
     if constexpr (RBT == 128)
         if (a.dl) {
             hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrDlState, 1, FX>), dim3(a.grid), dim3(RBT),
-                               a.lds, a.stream, a.st, *a.dl, a.tb, a.pm, a.rows, a.n_rows, a.T, a.x, a.hid, a.out,
-                               a.rb, a.n_data, a.arr, none);
+                               a.lds, a.stream, kern_args<InetNrDlState>(a));
             return;
         }
     hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(RBT), a.lds,
-                       a.stream, a.st, a.st, a.tb, a.pm, a.rows, a.n_rows, a.T, a.x, a.hid, a.out, a.rb, a.n_data,
-                       a.arr, none);
+                       a.stream, kern_args<InetNrState>(a));
 }
 
 // the multi-cell step: NC cells, pose input, runtime segment width (RBT = 0) or one fixed at compile time
 template <int S, int P, bool IR, int NC, int FX = 0, int RBT = 0>
 void launch_step_mc(const StepArgs& a) {
     hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, NC, FX>), dim3(a.grid), dim3(STEP_WAVE), a.lds,
-                       a.stream, a.st, a.st, a.tb, a.pm, a.rows, a.n_rows, a.T, a.x, a.hid, a.out, a.rb, a.n_data,
-                       a.arr, *a.cells);
+                       a.stream, kern_args<InetNrState>(a));
 }
 
 // every (P, IR, per-subband SNR) with a runtime segment width; plus, for segments of 32 lanes without IR or per-subband
