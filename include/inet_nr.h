@@ -148,7 +148,11 @@ typedef struct InetNrTables {
     int32_t M, C, G, NPRB, EQW, mcs_max;
     int32_t thr_monotone;     /* informational: thr_ref[0..mcs_max] non-decreasing (the kernels search its suffix
                                  minima, which give the highest passing MCS for any table) */
-    int32_t pad;
+    int32_t thr_ext;          /* 1: thr_ref holds two further words a, k: no TB of MCS m meets the BLER target at an
+                                 effective SINR (dB, OLLA offset included) below a + m / k, with a margin for the
+                                 float32 rounding of effective SINRs from -14 dB up, and none meets it below -14 dB;
+                                 the link adaptation starts its search there. 0: it starts at mcs_max. The results
+                                 are the same */
 } InetNrTables;
 
 /* Config constants of the step (derived on the host from NRConfig). */

@@ -26,7 +26,7 @@ class InetNrTables(C.Structure):
     _fields_ = [(n, P) for n in ("bler", "thr_ref", "se", "beta", "rate", "mcs_eq", "la_tbs", "la_ci0", "la_cwi",
                                  "la_ncb", "w", "logw", "wdb")] + \
                [(n, f32) for n in ("s0", "ds", "c0", "dc")] + \
-               [(n, i32) for n in ("M", "C", "G", "NPRB", "EQW", "mcs_max", "thr_monotone", "pad")]
+               [(n, i32) for n in ("M", "C", "G", "NPRB", "EQW", "mcs_max", "thr_monotone", "thr_ext")]
 
 
 class InetNrParams(C.Structure):

@@ -579,6 +579,8 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         }
         if (lane < MAX_M) s_thrs[lane] = lane <= tb.mcs_max ? v : __builtin_nanf("");
     }
+    // the line below the MCS floors where the link adaptation starts its search (none given: at the top)
+    const float la_a = tb.thr_ext ? tb.thr_ref[tb.M] : 0.0f, la_m1 = tb.thr_ext ? tb.thr_ref[tb.M + 1] : 0.0f;
     // log of the held PRB count by count of held RBGs, when every RBG has the same width: the log-sum-exp over the
     // held RBGs then adds exp(0) = 1 once per RBG, so it depends only on that count (s_lnw[n])
     if (lane <= S) s_lnw[lane] = lse_logw<S>(s_logw, lane >= 32 ? ~0u : ((1u << lane) - 1u));
@@ -1492,7 +1494,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                         __syncthreads();
                     }
 #pragma unroll 1
-                    for (int j = 0; j < rb; ++j) {
+                    for (int j = 0; j < R; ++j) {      // (the lanes past R hold no candidate)
                         float kj;
                         int vj;
                         if constexpr (W > 1) { kj = s_rkey[j]; vj = s_rval[j]; }
@@ -1733,9 +1735,32 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             s_la_f[lane] = la_lnw;
             s_la_f[CW + lane] = pm.olla ? olla : 0.0f;
             s_la_f[2 * CW + lane] = eff_md;
+            // Where the search starts. The EESM effective SINR of a row is at most its largest held SINR, so no MCS
+            // passes whose floor (the SINR that a TB of it needs at the least, PhyTables.la_floor) lies above that
+            // plus the OLLA offset, and the floors lie above the line la_a + m / la_m1, which also takes the
+            // float32 rounding of the log-sum-exp (from -14 dB; below, no MCS passes). Without a bound a robot at the
+            // cell edge walks down the whole table, a few candidates a round: default configuration 256 x 16 488 us
+            // without it, 385 us with it, 1024 x 32 570 and 462, three cells 1024 x 64 692 and 617. A search of the
+            // floors themselves from the tighter mean of the linear SINRs measured slower where few robots send (rl
+            // 4096 x 32 221 us against 217: LDS reads and a logarithm on the slot's serial chain).
             int top = tb.mcs_max, found_m = -1, tbs_found = 0;
             bool mine = tx_new;
             unsigned long long searching = __ballot(mine);
+            // (with a lane for every MCS of every searching robot the first round decides them all)
+            if (la_m1 != 0.0f && __popcll(searching) * (tb.mcs_max + 1) > STEP_WAVE) {
+                float b = eff_md;
+                if (pm.eesm) {
+                    b = -INFINITY;
+#pragma unroll
+                    for (int s = 0; s < S; ++s) {
+                        const float x = DL ? REF(s) + csi[s] : (REF(s) - sp) + csi[s];
+                        b = ((la_m >> s) & 1u) != 0u && x > b ? x : b;
+                    }
+                }
+                b = b + (pm.olla ? olla : 0.0f);
+                const float t = (clamp_min(b, -14.0f) - la_a) * la_m1;
+                top = nan || !(t < (float)tb.mcs_max) ? tb.mcs_max : (t > 0.0f ? (int)t : 0);
+            }
             auto more = [&]() -> bool {
                 if constexpr (W == 1) return searching != 0ull;
                 else return env_any(searching != 0ull);

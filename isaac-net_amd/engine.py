@@ -306,8 +306,10 @@ class HipNREngine:
         self._nsym_idx = {ns: i for i, ns in enumerate(nsyms)}
         la = [t.la_tables(cfg.nprb, ns, cfg.dmrs_re_per_prb, cfg.overhead_re_per_prb) for ns in nsyms]
         w = torch.tensor(cfg.subband_prbs, dtype=torch.float32)
+        line = t.la_line()
         host = {
-            "bler": torch.from_numpy(t.bler.reshape(-1)), "thr_ref": torch.from_numpy(t.thr_ref),
+            "bler": torch.from_numpy(t.bler.reshape(-1)),
+            "thr_ref": torch.from_numpy(np.concatenate([t.thr_ref, line or ()]).astype(np.float32)),
             "se": torch.from_numpy(t.se), "beta": torch.from_numpy(t.beta), "rate": torch.from_numpy(t.r),
             "mcs_eq": torch.from_numpy(t.mcs_eq.astype(np.int32)).reshape(-1),
             "la_tbs": torch.from_numpy(np.stack([x[0] for x in la])).reshape(-1),
@@ -323,6 +325,7 @@ class HipNREngine:
         c.s0, c.ds, c.c0, c.dc = t.s0, t.ds, t.c0, t.dc
         c.M, c.C, c.G, c.NPRB, c.EQW, c.mcs_max = t.M, t.C, t.G, cfg.nprb, t.mcs_eq.shape[1], t.mcs_max
         c.thr_monotone = int(bool(np.all(np.diff(t.thr_ref[:t.mcs_max + 1]) >= 0)))
+        c.thr_ext = int(line is not None)
         self._ctab = c
         if self.dl:                                   # the same tables with the DL MCS cap
             cd = _lib.InetNrTables()

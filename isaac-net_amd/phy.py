@@ -194,6 +194,31 @@ class PhyTables:
         m_ = np.arange(M)
         self.thr_ref = (self.thr[m_, i0] * (_f32(1) - wi) + self.thr[m_, i0 + 1] * wi).astype(_f32)
 
+    def la_floor(self):
+        """Per MCS the SINR (dB) below which no TB meets the BLER target, whatever its code-block size and count [M]:
+        the SNR grid point before the first one where some code-block size's BLER is under the target. Below it
+        all four corners of a bilinear lookup exceed the target, and a TB of several blocks fails more often than
+        one block (margins: 1e-6 in BLER and 1e-3 dB, above the float32 rounding of the lookup and of the floor)."""
+        ok = self.bler.min(1) < self.target + 1e-6
+        j = np.where(ok.any(-1), ok.argmax(-1), self.G)
+        f = self.s0 + self.ds * (j - 1.0) - 1e-3
+        return np.where(j <= 1, -np.inf, np.where(j >= self.G, np.inf, f))
+
+    def la_line(self):
+        """(a, k) float32 with a + m / k below every MCS's floor, less the float32 rounding of an EESM effective SINR:
+        at most 1e-5 beta (linear), in dB at -14 dB or more; None where some MCS has no floor or one below -14 dB, or
+        the floors do not rise."""
+        f = self.la_floor()
+        ok = np.isfinite(f)
+        if ok.sum() < 2 or (f < -13.5).any():
+            return None
+        m = np.arange(self.M)[ok]
+        slope = float(np.polyfit(m, f[ok], 1)[0])
+        if slope <= 1e-3:
+            return None
+        margin = 10 * math.log10(1 + 1e-5 * float(self.beta.max()) / 10 ** -1.4) + 2e-3
+        return _f32((f[ok] - slope * m).min() - margin), _f32(1 / slope)
+
     def tbs_all(self, n_prb, nsym, dmrs=12, oh=0):
         """TBS (bits) of every MCS for PRB counts n_prb [...] -> [..., M] int64."""
         n = np.asarray(n_prb, dtype=np.float64)[..., None]
