@@ -516,6 +516,18 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
         }
     }
+    // the processes by state, a bit each: undecoded (1), free (0); the rest wait for their HARQ-ACK (2, DL)
+    uint32_t m_pend = 0u, m_free = 0u;
+    auto harq_masks = [&]() {
+        m_pend = 0u; m_free = 0u;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const int stp = hm_state(hmeta[p]);
+            m_pend |= stp == 1 ? 1u << p : 0u;
+            m_free |= stp == 0 ? 1u << p : 0u;
+        }
+    };
+    harq_masks();
     // Rician state of every robot-cell link c ([E][NC][R]): specular phasor, K target kk, ramp start kf and slot kg
     float sp_re[NC], sp_im[NC], kk[NC], kf[NC];
     int kg[NC];
@@ -773,7 +785,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         int a = sent;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            bool own = hm_state(hmeta[p]) == 1 && hhi[p] > floor_;
+            bool own = ((m_pend >> p) & 1u) != 0u && hhi[p] > floor_;
             int lo = hlo[p] > floor_ ? hlo[p] : floor_;
             if (own && lo < a) a = lo;
         }
@@ -866,6 +878,8 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
 #pragma unroll
             for (int p = 0; p < P; ++p)
                 if (hm_state(hmeta[p]) == 1) hmeta[p] = hm_pack(0, hm_ntx(hmeta[p]), hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
+            m_free |= m_pend;
+            m_pend = 0u;
         } else {
 #pragma unroll
             for (int p = 0; p < P; ++p) {
@@ -1018,6 +1032,11 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     const int last_ul_row = m_ul ? 63 - __builtin_clzll(m_ul) : -1;
     const int last_h_row = m_h ? 63 - __builtin_clzll(m_h) : -1;
     const bool iid = m_corr == 0ull;
+    // whether the gains have to be formed anew at the next UL slot: a fading state has moved since the last one (a step
+    // of i.i.d. draws begins without the state, and every robot draws at the step's last UL slot)
+    bool new_gain = !iid || read_h || !pm.fading;
+    int ack_cur = 0;                                   // the in-order pointer, as of the last transmission
+    bool ack_known = false;
     INET_PH(0);                                    // prologue: tables, state loads, arrivals, radio
     // ================================================================ slot loop
     for (int k = 0; k < n_rows; ++k) {
@@ -1040,14 +1059,12 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             // (robot, link) pairs are dealt round-robin over the 64 lanes, each pair's two normals land in the
             // robot's LDS column (s_x), and the robot then updates its own state. Normal j = 2 NC S r + 2 q + {0, 1}
             // (link q = c S + s of cell c and subband s; real, imaginary part) uses hash elements 2j, 2j + 1.
-            bool busy = false;
-#pragma unroll
-            for (int p = 0; p < P; ++p) busy |= hm_state(hmeta[p]) == 1;
-            busy |= (enq - sent) > 0;
+            const bool busy = m_pend != 0u || (enq - sent) > 0;
             // (the DL draws every robot's gain at its CQI rows, which set the CSI of every robot)
             const bool full = !iid || (DL ? (row.flags & 1) != 0 : (k == last_ul_row || k == last_h_row));
             const bool draw = act && (full || busy);
             const unsigned long long need = __ballot(draw);              // (per wave: each draws its own robots)
+            new_gain |= need != 0ull;
             float* const s_z = s_x;
             // the env's key of this slot, and the hash input of the robot's first element (robot r's normals start at
             // element 2 NC S r, hash element 2 (2 NC S r) = 4 NC S r)
@@ -1298,26 +1315,34 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         const int unsent = enq - sent;
         if constexpr (DL) {
             // DL processes whose HARQ-ACK has reached the gNB become free (mac.py:243)
+            constexpr uint32_t ALL_P = P >= 32 ? ~0u : (1u << P) - 1u;
+            if (__ballot((m_pend | m_free) != ALL_P) != 0ull) {
 #pragma unroll
-            for (int p = 0; p < P; ++p)
-                if (hm_state(hmeta[p]) == 2 && hrdy[p] <= g)
-                    hmeta[p] = hm_pack(0, hm_ntx(hmeta[p]), hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
+                for (int p = 0; p < P; ++p)
+                    if (hm_state(hmeta[p]) == 2 && hrdy[p] <= g) {
+                        hmeta[p] = hm_pack(0, hm_ntx(hmeta[p]), hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
+                        m_free |= 1u << p;
+                    }
+            }
         } else {
             // grants (UlMac._pre_slot_lumped)
             if (row.flags & 16) bsr = bsr > 1 ? bsr : 1;
             if (sr_t >= 0 && g - sr_t >= pv.sr_delay) { bsr = bsr > 1 ? bsr : 1; sr_t = -1; }
         }
         // candidates: the retransmission ready first (lowest ready slot, then lowest process), the lowest free process
-        int rx_p = 0, p_new = 0;
+        int rx_p = 0;
         int best_rdy = 0x7fffffff;
-        bool has_rx = false, any_free = false, pending = false;
+        if (__ballot(m_pend != 0u) != 0ull) {
 #pragma unroll
-        for (int p = P - 1; p >= 0; --p) {
-            int stp = hm_state(hmeta[p]);
-            if (stp == 1 && hrdy[p] <= g && hrdy[p] <= best_rdy) { best_rdy = hrdy[p]; rx_p = p; has_rx = true; }
-            if (stp == 0) { any_free = true; p_new = p; }
-            if (stp == 1) pending = true;
+            for (int p = P - 1; p >= 0; --p) {
+                const int rdy = ((m_pend >> p) & 1u) != 0u ? hrdy[p] : 0x7fffffff;
+                if (rdy <= best_rdy) { best_rdy = rdy; rx_p = p; }
+            }
         }
+        // (the slot numbers stay below 2^31 - 1: the largest bid stands for none pending)
+        bool has_rx = best_rdy <= g;
+        const bool any_free = m_free != 0u, pending = m_pend != 0u;
+        const int p_new = any_free ? __builtin_ctz(m_free) : 0;
         const int need = DL ? unsent : (bsr < unsent ? bsr : unsent);
         bool new_el = any_free && need > 0 && !has_rx && act;
         has_rx = has_rx && act;
@@ -1339,8 +1364,18 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         float* const s_met = s_x;
         float* const s_eo = s_x + S * CW;
         float* const s_rt = s_lin;
+        const bool bid0 = has_rx || new_el;
+        // a slot in which nobody bids (of the wavefront; W > 1: of the env) passes over the scheduler altogether: its
+        // S winner searches are a serial chain of lane exchanges (W > 1: of barriers). Of the slots of 16384 x 128
+        // (0.01 TBs per robot and slot) most are such: 2526 -> 1964 us; UL and DL 4096 x 32 566 -> 511 us
+        bool any_bid;
+        if constexpr (W == 1) any_bid = __ballot(bid0) != 0ull;
+        else any_bid = env_any(bid0);
+        int cnt = 0;
+        uint32_t won = 0;
+        auto metric_of = [&](int s) -> float { return s_met[s * CW + lane]; };
+        if (any_bid) {
         {
-            const bool bid0 = has_rx || new_el;
             if (bid0) {
 #pragma unroll
                 for (int s = 0; s < S; ++s) {
@@ -1455,7 +1490,6 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             }
             __syncthreads();
         }
-        auto metric_of = [&](int s) -> float { return s_met[s * CW + lane]; };
         INET_PH(2);                                // SR / CQI, grants, candidates, estimate, MCS, rate, metric
         // retransmission admission (mac.py:300-313): rank by the metric sum inside each scheduler, admit while the RBG
         // counts fit (the segment's total fitting implies every cell's)
@@ -1556,9 +1590,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             rate[s] = s_rt[s * CW + lane];
             asm volatile("" : "+v"(mrow[s]), "+v"(rate[s]));
         }
-        int cnt = 0;
         float left = (float)need;
-        uint32_t won = 0;
         // pf_update "rbg" (mac.py:325-329, 526-532): the metric of RBG s is rate_s / max(base + wwin got, 1e-9) with
         // base = (1 - wwin) avg and got the rate of the RBGs this robot won so far in the slot
         const float pf_base = pv.pf_a * avg;
@@ -1603,6 +1635,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                 left = left - (sel ? rate[s] : 0.0f);
             }
         }
+        }
         INET_PH(4);                                // RBG-by-RBG allocation
         const int n_sb = __popc(won);
         float n_prb = 0.f;
@@ -1611,6 +1644,20 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         const bool tx_rx = has_rx && n_sb == rx_nsb && n_sb > 0;
         const bool tx_new = new_el && n_sb > 0;
         const bool tx = tx_rx || tx_new;
+        bool any_tx = false, any_new = false;          // (W > 1: of the env, so that every wave reaches the barriers)
+        if (any_bid) {
+            if constexpr (W == 1) {
+                any_tx = __ballot(tx) != 0ull;
+                any_new = __ballot(tx_new) != 0ull;
+            } else {
+                int a[W], any = 0;
+                xchgw((__ballot(tx) != 0ull ? 1 : 0) | (__ballot(tx_new) != 0ull ? 2 : 0), a);
+#pragma unroll
+                for (int w = 0; w < W; ++w) any |= a[w];
+                any_tx = (any & 1) != 0;
+                any_new = (any & 2) != 0;
+            }
+        }
         // power split (mac_ul.py:173-180): PUSCH power spread over n_prb PRBs, at least the power-control backoff
         const float sp0 = pm.whole_band ? pv.wb_db : 10.0f * log10_clamped(clamp_min(n_prb / pv.snr_ref_prbs, 1e-3f));
         const float sp = use_pc ? (sp0 > pc ? sp0 : pc) : sp0;
@@ -1677,9 +1724,6 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         };
         // ---- link adaptation for new TBs (phy.select_mcs): the highest MCS meeting the BLER target ----
         int mcs_new = 0, tbs_new = 0;
-        bool any_new;                                  // (W = 2: both waves enter, the search has barriers)
-        if constexpr (W == 1) any_new = __ballot(tx_new) != 0ull;
-        else any_new = env_any(tx_new);
         if (any_new) {
             // the RBGs the MCS is searched over: the held ones; ul_amc_alloc "previous" with whole-band power, every
             // RBG (mac.py:396)
@@ -1822,29 +1866,38 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         cap_b = cap_b > 1 ? cap_b : 1;
         const int byt_new = cap_b < unsent ? cap_b : unsent;
         // ---- bind TBs to HARQ processes (mac.py:407-426) ----
+        // The process's words as this transmission has them: a new TB's, or those of the retransmitting process. The
+        // arrays are read only in wavefronts that retransmit and written once, after decoding.
         const int p_tx = tx_rx ? rx_p : p_new;
-        int mcs = 0, tbs = 0, ntx = 1, lo_tx = 0, hi_tx = 0;
+        uint32_t meta_tx = hm_pack(1, 0, mcs_new, n_sb);
+        int tbs = tbs_new, lo_tx = sent, hi_tx = sent + byt_new;
         float comb_p = 0.f, lexp_p = -INFINITY, nrb_p = 0.f;
+        if (__ballot(tx_rx) != 0ull) {
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            if (p == p_tx) {
-                if (tx_new) {
-                    hlo[p] = sent; hhi[p] = sent + byt_new; htbs[p] = tbs_new;
-                    hmeta[p] = hm_pack(1, 0, mcs_new, n_sb);
-                    hcomb[p] = 0.f;
-                    if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
-                }
-                mcs = hm_mcs(hmeta[p]); tbs = htbs[p]; ntx = hm_ntx(hmeta[p]) + 1;
-                comb_p = hcomb[p]; lo_tx = hlo[p]; hi_tx = hhi[p];
-                if constexpr (IR) { lexp_p = hlexp[p]; nrb_p = hnrb[p]; }
+            for (int p = 0; p < P; ++p) {
+                const bool m = tx_rx && p == rx_p;
+                meta_tx = m ? hmeta[p] : meta_tx;
+                tbs = m ? htbs[p] : tbs;
+                lo_tx = m ? hlo[p] : lo_tx;
+                hi_tx = m ? hhi[p] : hi_tx;
+                comb_p = m ? hcomb[p] : comb_p;
+                if constexpr (IR) { lexp_p = m ? hlexp[p] : lexp_p; nrb_p = m ? hnrb[p] : nrb_p; }
             }
         }
+        const int ntx = hm_ntx(meta_tx) + 1;
+        int mcs = hm_mcs(meta_tx);
         mcs = mcs < tb.M ? mcs : tb.M - 1;
         if (tx_new) sent = sent + byt_new;
         // ---- actual channel of this slot: fading gain per subband; in the UL it becomes the CSI (mac_ul.py:229-236)
+        // (DL: read by the decode only; UL, one cell: the same values again where no robot of the wavefront has drawn
+        // since the last data slot)
         float gn[DL ? S : 1];
-        if constexpr (DL) gains_of(gn);
-        else gains_of(csi);
+        if constexpr (DL) {
+            if (any_tx) gains_of(gn);
+        } else {
+            if (MC || new_gain || kl) gains_of(csi);
+            new_gain = false;
+        }
         // ---- several cells: same-slot UL interference (NRNet._ul_ici, nr_engine.py:799-816) ----
         // Every robot that transmits adds, at each other cell c and RBG s it holds, its received power
         // 10^((((pg_c + ue_tx) - ref_db) - split + gain_cs) / 10) (mW per PRB). Each lane writes its NC S terms (zeros
@@ -1930,9 +1983,6 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         // ---- decoding on the actual channel (mac.py:428-454, mac_ul.py:185-192) ----
         bool ok = false, fail = false, exh = false;
         float comb = comb_p, lexp = lexp_p, nrb = nrb_p;
-        bool any_tx;                                   // (W = 2: both waves enter, the EESM has barriers)
-        if constexpr (W == 1) any_tx = __ballot(tx) != 0ull;
-        else any_tx = env_any(tx);
         if (any_tx) {
             const float beta = s_beta[mcs], rbeta = s_rbeta[mcs];
             bool nan = false;
@@ -1995,25 +2045,29 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             rdy_fail = rdy_ok;
             st_ok = 2;
         }
+        if (any_tx) {
+            const bool again = exh && !pm.harq_drop;     // RLC AM: the TB starts over after rlc_retx slots
+            const int st_tx = ok ? st_ok : (exh && pm.harq_drop ? 0 : 1);
+            const uint32_t nm = hm_pack(st_tx, again ? 0 : ntx, hm_mcs(meta_tx), hm_nsb(meta_tx));
+            const int nrdy = ok ? rdy_ok : (again ? g + pv.rlc_retx : rdy_fail);
+            const float ncomb = again ? 0.f : comb;
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            if (p == p_tx && tx) {
-                int stp = hm_state(hmeta[p]);
-                int ntxp = ntx;
-                if (ok) { stp = st_ok; hrdy[p] = rdy_ok; }
-                hcomb[p] = comb;
-                if constexpr (IR) { hlexp[p] = lexp; hnrb[p] = nrb; }
-                if (fail) hrdy[p] = rdy_fail;
-                if (exh) {
-                    if (pm.harq_drop) stp = 0;
-                    else {
-                        ntxp = 0; hcomb[p] = 0.f;
-                        if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
-                        hrdy[p] = g + pv.rlc_retx;
-                    }
+            for (int p = 0; p < P; ++p) {
+                const bool m = tx && p == p_tx;
+                hmeta[p] = m ? nm : hmeta[p];
+                hrdy[p] = m ? nrdy : hrdy[p];
+                hcomb[p] = m ? ncomb : hcomb[p];
+                hlo[p] = m ? lo_tx : hlo[p];
+                hhi[p] = m ? hi_tx : hhi[p];
+                htbs[p] = m ? tbs : htbs[p];
+                if constexpr (IR) {
+                    hlexp[p] = m ? (again ? -INFINITY : lexp) : hlexp[p];
+                    hnrb[p] = m ? (again ? 0.f : nrb) : hnrb[p];
                 }
-                hmeta[p] = hm_pack(stp, ntxp, hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
             }
+            const uint32_t bit = tx ? 1u << p_tx : 0u;
+            m_pend = (m_pend & ~bit) | (st_tx == 1 ? bit : 0u);
+            m_free = (m_free & ~bit) | (st_tx == 0 ? bit : 0u);
         }
         // ---- OLLA, BSR, PF average, RR (mac.py:479-485, mac_ul.py:229-236, mac.py:534-554) ----
         if (pm.olla) olla = clampf((olla + pv.olla_up * (ok ? 1.0f : 0.0f)) - pv.olla_dn * (fail ? 1.0f : 0.0f),
@@ -2030,6 +2084,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         }
         if (pm.sched == 2 && tx) last_tx = g;
         // ---- counters ----
+        if (any_tx) {
         c_new += tx_new; c_retx += tx_rx; c_ok += ok; c_fail += fail; c_exh += exh;
         c_bytes_ok += served; c_bytes_new += tx_new ? byt_new : 0; c_new_pend += (tx_new && pending);
         c_prb += tx ? (int)n_prb : 0;
@@ -2039,13 +2094,15 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             atomicAdd(&my_hist[HB + kh], 1);
             atomicAdd(&my_hist[(ok ? 0 : 2 * HB) + kh], 1);
         }
+        }
         // ---- RLC in-order pointer of this slot ----
         if constexpr (DL) {
             // the DL link resolves its frames as the pointer moves (no per-slot history in LDS): under RLC UM the
             // frames an exhausted TB overlaps are lost (mac.py:474-477), then the frames the in-order pointer has
             // passed complete at this slot (mac.py:500-503). Frames before nf are lost or completed, and no
             // completed frame overlaps an undecoded TB, so both scans start at nf.
-            if (act) {
+            // (no transmission of the wavefront since the last data slot: the pointer and the frames stay as they were)
+            if ((any_tx || !ack_known) && act) {
                 if (pm.harq_drop && exh) {
                     for (int f = nf; f < qlen; ++f) {
                         const int fr = f * R;
@@ -2065,8 +2122,11 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     sto(lk.q_fin + fr, o_fr0, g);
                 }
             }
+            ack_known = true;
         } else if (n_ul < n_ul_max) {            // (UL: recorded, completion replayed in the epilogue)
-            ack_l[n_ul * CW + lane] = ack_ptr();
+            if (MC || any_tx || !ack_known) ack_cur = ack_ptr();
+            ack_known = true;
+            ack_l[n_ul * CW + lane] = ack_cur;
             if (pm.harq_drop) {
                 exlo_l[n_ul * CW + lane] = exh ? lo_tx : 0;
                 exhi_l[n_ul * CW + lane] = exh ? hi_tx : 0;
