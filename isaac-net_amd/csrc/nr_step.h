@@ -483,9 +483,13 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     int sent = 0, floor_ = 0, bsr = 0, sr_t = -1, last_tx = -1, enq = 0, qlen = 0;
     float olla = 0.f, avg = 100.f;
     float csi[S], hr[NCS], hi[NCS];
+    // per HARQ process: its state word, first byte and ready slot. The words that only a transmission of the process
+    // touches (its last byte, TBS, combined SINR, IR sums) stay in memory: a retransmission reads them, a transmission
+    // writes them. In registers they took 3 P (IR: 5 P) of the 256, spilled at 16 processes and with two waves per env
+    // (120 and 108 B per lane of scratch, now 0 and 52), and were read and written whole: 4096 x 100 at 16 processes
+    // 1563 -> 1371 us, 16384 x 128 1964 -> 1712, rl 4096 x 32 210.5 -> 203.6, HARQ-IR 1024 x 16 243 -> 226.
     uint32_t hmeta[P];
-    int hlo[P], hhi[P], hrdy[P], htbs[P];
-    float hcomb[P], hlexp[IR ? P : 1], hnrb[IR ? P : 1];
+    int hlo[P], hrdy[P];
     const bool read_h = pm.fading && !(n_rows > 0 && (rows[0].flags & 4) && rows[0].rho == 0.0f);
     // (lanes without a robot read a clamped, valid address and discard the value: the loads are branch-free)
     sent = ldo(lk.sent, o_r); floor_ = ldo(lk.floor_, o_r);
@@ -505,29 +509,25 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         hr[q] = 0.f; hi[q] = 0.f;
         if (read_h && act) { hr[q] = ldo(st.h_re + q * R, o_hr0); hi[q] = ldo(st.h_im + q * R, o_hr0); }
     }
+    // the undecoded processes that hold back the in-order pointer: their bytes reach past the floor
+    uint32_t m_own = 0u;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const int pr = p * R;
-        hmeta[p] = ldo(lk.h_meta + pr, o_pr); hlo[p] = ldo(lk.h_lo + pr, o_pr); hhi[p] = ldo(lk.h_hi + pr, o_pr);
-        hrdy[p] = ldo(lk.h_ready + pr, o_pr); htbs[p] = ldo(lk.h_tbs + pr, o_pr); hcomb[p] = ldo(lk.h_comb + pr, o_pr);
-        if constexpr (IR) { hlexp[p] = ldo(lk.h_lexp + pr, o_pr); hnrb[p] = ldo(lk.h_nrb + pr, o_pr); }
-        if (!act) {
-            hmeta[p] = 0u; hlo[p] = 0; hhi[p] = 0; hrdy[p] = 0; htbs[p] = 0; hcomb[p] = 0.f;
-            if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
-        }
+        hmeta[p] = ldo(lk.h_meta + pr, o_pr); hlo[p] = ldo(lk.h_lo + pr, o_pr); hrdy[p] = ldo(lk.h_ready + pr, o_pr);
+        const int hi = ldo(lk.h_hi + pr, o_pr);
+        if (!act) { hmeta[p] = 0u; hlo[p] = 0; hrdy[p] = 0; }
+        m_own |= act && hi > floor_ ? 1u << p : 0u;
     }
     // the processes by state, a bit each: undecoded (1), free (0); the rest wait for their HARQ-ACK (2, DL)
     uint32_t m_pend = 0u, m_free = 0u;
-    auto harq_masks = [&]() {
-        m_pend = 0u; m_free = 0u;
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int stp = hm_state(hmeta[p]);
-            m_pend |= stp == 1 ? 1u << p : 0u;
-            m_free |= stp == 0 ? 1u << p : 0u;
-        }
-    };
-    harq_masks();
+    for (int p = 0; p < P; ++p) {
+        const int stp = hm_state(hmeta[p]);
+        m_pend |= stp == 1 ? 1u << p : 0u;
+        m_free |= stp == 0 ? 1u << p : 0u;
+    }
+    m_own &= m_pend;
     // Rician state of every robot-cell link c ([E][NC][R]): specular phasor, K target kk, ramp start kf and slot kg
     float sp_re[NC], sp_im[NC], kk[NC], kf[NC];
     int kg[NC];
@@ -785,7 +785,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         int a = sent;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            bool own = ((m_pend >> p) & 1u) != 0u && hhi[p] > floor_;
+            const bool own = ((m_own >> p) & 1u) != 0u;
             int lo = hlo[p] > floor_ ? hlo[p] : floor_;
             if (own && lo < a) a = lo;
         }
@@ -863,7 +863,8 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     const int qs = ldo(lk.q_start + f * R, o_fr0), qe = ldo(lk.q_end + f * R, o_fr0);
                     bool ov = false;
 #pragma unroll
-                    for (int p = 0; p < P; ++p) ov |= hm_state(hmeta[p]) == 1 && qs < hhi[p] && qe > hlo[p];
+                    for (int p = 0; p < P; ++p)
+                        if ((m_pend >> p) & 1u) ov |= qs < ldo(lk.h_hi + p * R, o_pr0) && qe > hlo[p];
                     if (ov) mk |= 1ull << f;
                 }
             }
@@ -880,13 +881,14 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                 if (hm_state(hmeta[p]) == 1) hmeta[p] = hm_pack(0, hm_ntx(hmeta[p]), hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
             m_free |= m_pend;
             m_pend = 0u;
+            m_own = 0u;
         } else {
 #pragma unroll
             for (int p = 0; p < P; ++p) {
                 if (hm_state(hmeta[p]) == 1) {
                     hmeta[p] = hm_pack(1, 0, hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
-                    hcomb[p] = 0.f;
-                    if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
+                    sto(lk.h_comb + p * R, o_pr0, 0.f);
+                    if constexpr (IR) { sto(lk.h_lexp + p * R, o_pr0, -INFINITY); sto(lk.h_nrb + p * R, o_pr0, 0.f); }
                 }
             }
         }
@@ -1644,6 +1646,15 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         const bool tx_rx = has_rx && n_sb == rx_nsb && n_sb > 0;
         const bool tx_new = new_el && n_sb > 0;
         const bool tx = tx_rx || tx_new;
+        // a retransmission's words from memory: asked for here, used after the link adaptation of the new TBs
+        const LS& lv = [&]() -> const LS& { if constexpr (DL) return args.lk; else return args.st; }();
+        int tbs_rx = 0, hi_rx = 0;
+        float comb_p = 0.f, lexp_p = -INFINITY, nrb_p = 0.f;
+        if (tx_rx) {
+            const uint32_t o = o_pr0 + (uint32_t)(rx_p * R) * 4u;
+            tbs_rx = ldo(lv.h_tbs, o); hi_rx = ldo(lv.h_hi, o); comb_p = ldo(lv.h_comb, o);
+            if constexpr (IR) { lexp_p = ldo(lv.h_lexp, o); nrb_p = ldo(lv.h_nrb, o); }
+        }
         bool any_tx = false, any_new = false;          // (W > 1: of the env, so that every wave reaches the barriers)
         if (any_bid) {
             if constexpr (W == 1) {
@@ -1866,23 +1877,14 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         cap_b = cap_b > 1 ? cap_b : 1;
         const int byt_new = cap_b < unsent ? cap_b : unsent;
         // ---- bind TBs to HARQ processes (mac.py:407-426) ----
-        // The process's words as this transmission has them: a new TB's, or those of the retransmitting process. The
-        // arrays are read only in wavefronts that retransmit and written once, after decoding.
+        // the process's words as this transmission has them: a new TB's, or those of the retransmitting process
         const int p_tx = tx_rx ? rx_p : p_new;
         uint32_t meta_tx = hm_pack(1, 0, mcs_new, n_sb);
-        int tbs = tbs_new, lo_tx = sent, hi_tx = sent + byt_new;
-        float comb_p = 0.f, lexp_p = -INFINITY, nrb_p = 0.f;
+        int lo_tx = sent;
+        const int tbs = tx_rx ? tbs_rx : tbs_new, hi_tx = tx_rx ? hi_rx : sent + byt_new;
         if (__ballot(tx_rx) != 0ull) {
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const bool m = tx_rx && p == rx_p;
-                meta_tx = m ? hmeta[p] : meta_tx;
-                tbs = m ? htbs[p] : tbs;
-                lo_tx = m ? hlo[p] : lo_tx;
-                hi_tx = m ? hhi[p] : hi_tx;
-                comb_p = m ? hcomb[p] : comb_p;
-                if constexpr (IR) { lexp_p = m ? hlexp[p] : lexp_p; nrb_p = m ? hnrb[p] : nrb_p; }
-            }
+            meta_tx = tx_rx ? sel_of(hmeta, rx_p) : meta_tx;
+            lo_tx = tx_rx ? sel_of(hlo, rx_p) : lo_tx;
         }
         const int ntx = hm_ntx(meta_tx) + 1;
         int mcs = hm_mcs(meta_tx);
@@ -2056,17 +2058,20 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                 const bool m = tx && p == p_tx;
                 hmeta[p] = m ? nm : hmeta[p];
                 hrdy[p] = m ? nrdy : hrdy[p];
-                hcomb[p] = m ? ncomb : hcomb[p];
                 hlo[p] = m ? lo_tx : hlo[p];
-                hhi[p] = m ? hi_tx : hhi[p];
-                htbs[p] = m ? tbs : htbs[p];
+            }
+            if (tx) {
+                const uint32_t o = o_pr0 + (uint32_t)(p_tx * R) * 4u;
+                sto(lv.h_comb, o, ncomb);
+                if (tx_new) { sto(lv.h_hi, o, hi_tx); sto(lv.h_tbs, o, tbs); }
                 if constexpr (IR) {
-                    hlexp[p] = m ? (again ? -INFINITY : lexp) : hlexp[p];
-                    hnrb[p] = m ? (again ? 0.f : nrb) : hnrb[p];
+                    sto(lv.h_lexp, o, again ? -INFINITY : lexp);
+                    sto(lv.h_nrb, o, again ? 0.f : nrb);
                 }
             }
             const uint32_t bit = tx ? 1u << p_tx : 0u;
             m_pend = (m_pend & ~bit) | (st_tx == 1 ? bit : 0u);
+            m_own = (m_own & ~bit) | (st_tx == 1 && hi_tx > floor_ ? bit : 0u);
             m_free = (m_free & ~bit) | (st_tx == 0 ? bit : 0u);
         }
         // ---- OLLA, BSR, PF average, RR (mac.py:479-485, mac_ul.py:229-236, mac.py:534-554) ----
@@ -2298,10 +2303,15 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     sent = sent > floor_ ? sent : floor_;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        if (hm_state(hmeta[p]) == 1 && hhi[p] <= floor_ && hhi[p] > hlo[p]) {
-            hmeta[p] = hm_pack(0, 0, hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
-            hrdy[p] = 0; hcomb[p] = 0.f;
-            if constexpr (IR) { hlexp[p] = -INFINITY; hnrb[p] = 0.f; }
+        if (((m_pend >> p) & 1u) != 0u) {
+            const int hi = ldo(lk.h_hi + p * R, o_pr0);
+            if (hi <= floor_) m_own &= ~(1u << p);
+            if (hi <= floor_ && hi > hlo[p]) {
+                hmeta[p] = hm_pack(0, 0, hm_mcs(hmeta[p]), hm_nsb(hmeta[p]));
+                hrdy[p] = 0;
+                sto(lk.h_comb + p * R, o_pr0, 0.f);
+                if constexpr (IR) { sto(lk.h_lexp + p * R, o_pr0, -INFINITY); sto(lk.h_nrb + p * R, o_pr0, 0.f); }
+            }
         }
     }
     if constexpr (!DL) {
@@ -2322,9 +2332,9 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         sent -= b; enq -= b; floor_ = 0;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            const int64_t lo = (int64_t)hlo[p] - b, hi = (int64_t)hhi[p] - b;
+            const int64_t lo = (int64_t)hlo[p] - b, hi = (int64_t)ldo(lk.h_hi + p * R, o_pr0) - b;
             hlo[p] = (int)(lo < -(1ll << 30) ? -(1ll << 30) : lo);
-            hhi[p] = (int)(hi < -(1ll << 30) ? -(1ll << 30) : hi);
+            sto(lk.h_hi + p * R, o_pr0, (int)(hi < -(1ll << 30) ? -(1ll << 30) : hi));
         }
         for (int f = 0; f < kept; ++f) {
             const int fr = f * R;
@@ -2380,9 +2390,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const int pr = p * R;
-            sto(lk.h_meta + pr, o_pr, hmeta[p]); sto(lk.h_lo + pr, o_pr, hlo[p]); sto(lk.h_hi + pr, o_pr, hhi[p]);
-            sto(lk.h_ready + pr, o_pr, hrdy[p]); sto(lk.h_tbs + pr, o_pr, htbs[p]); sto(lk.h_comb + pr, o_pr, hcomb[p]);
-            if constexpr (IR) { sto(lk.h_lexp + pr, o_pr, hlexp[p]); sto(lk.h_nrb + pr, o_pr, hnrb[p]); }
+            sto(lk.h_meta + pr, o_pr, hmeta[p]); sto(lk.h_lo + pr, o_pr, hlo[p]); sto(lk.h_ready + pr, o_pr, hrdy[p]);
         }
         if constexpr (DL) {
             // NRNet.dl_newest (absolute) and the step outputs dl_newest (env clock) and dl_queue_len
