@@ -385,6 +385,7 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
     inet::StepArgs a{*st, dl, cells, t, p, rows, n_rows, n_hist, arr ? *arr : none, T, x, cur_hid, *out, rb,
                      (unsigned)((p.E + envs_pw - 1) / envs_pw),
                      inet::step_lds_bytes(n_hist, p.harq_drop, rb, p.max_tx, cells ? cells->C : 1, p.S),
+                     inet::step_lds_bytes(0, p.harq_drop, rb, p.max_tx),
                      (hipStream_t)stream};
     // several cells: the static LDS grows with the cells (each lane's fading normals, 2 NC S floats, the
     // interference pairs and every robot's PSD at each cell; under 16 KiB besides) and must fit the CU's 160 KiB

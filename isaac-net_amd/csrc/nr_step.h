@@ -330,6 +330,12 @@ DEV const StepKernArgs<LS>& args_again() {
     return *(const StepKernArgs<LS>*)p;
 }
 
+// The builds that complete frames as the in-order pointer passes them: the common configuration in one cell (no losses to
+// place among the slots). The history's 4 B per lane and slot bound the workgroups of a CU, and its replay costs
+// frames x slots: 16384 x 128 (20 UL slots) 1712 -> 1558 us, the default configuration 1024 x 32 (20 UL slots, long
+// queues) 434 -> 413, 4096 x 100 1371 -> 1355, rl 4096 x 32 205.8 -> 204.4 (same card).
+constexpr bool step_walks(int NC, int FX) { return NC == 1 && FX != 0; }
+
 // RBT: the segment width when it is fixed at compile time (0: the runtime argument rb).
 // LS: the link whose MAC state and queue the kernel runs: InetNrState (the UL; lk is st) or InetNrDlState (the DL
 // of NRConfig(dl=True): CQI reports and DL data slots with the DlMac hooks; it reads the shared state of st and writes
@@ -348,8 +354,9 @@ DEV const StepKernArgs<LS>& args_again() {
 // bit for bit; fx_profile), FX = 2 for the same without the Rician phasor: those switches become compile-time constants, which removes their tests from the slot loop and the scalar registers that
 // hold them.
 // Minimum waves per SIMD (the register budget): 2, and 3 for the two-wave FX = 2 build (envs of 65..128 robots at the
-// common configuration: 168 VGPRs with 104 B per lane of spills, measured 7% faster than 193 VGPRs at 2 waves on
-// 16384 x 128; 4 waves, at 128 VGPRs, spill enough to be 30% slower); 1 with several cells.
+// common configuration, 8 RBGs and processes: 168 VGPRs with 72 B per lane of spills, 1558 us on 16384 x 128 against
+// 1867 for 204 VGPRs at 2 waves; 4 waves, at 128 VGPRs and 232 B, take 2427. 13 RBGs with 16 processes at 3 waves spill
+// 332 B: 4096 x 100 1951 us against 1353); 1 with several cells.
 template <int S, int P, bool IR, bool VREF, int RBT, class LS, int NC, int FX = 0>
 __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1),
                              NC > 1 ? 1 : ((RBT == 128 && FX == 2) ? 3 : 2)) void nr_step_kernel(
@@ -376,6 +383,11 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     // the link whose MAC state the kernel runs: the UL link is the shared state itself (one set of pointers)
     const LS& lk = [&]() -> const LS& { if constexpr (DL) return args.lk; else return args.st; }();
     constexpr bool MC = NC > 1;
+    // Frames complete as the in-order pointer passes them (one cell, RLC AM): the end of the first frame not completed
+    // is in a register, that of the next one on its way, and a completion writes its slot. The other builds record
+    // the pointer of every UL slot in LDS and replay it over the queue at the end, where losses have their place among
+    // the slots.
+    constexpr bool WALK = step_walks(NC, FX);
     static_assert(!(MC && (DL || VREF)), "several cells: the UL with pose input");
     constexpr int W = RBT > STEP_WAVE ? RBT / STEP_WAVE : 1;   // wavefronts per env (1, 2 or 4)
     static_assert(W == 1 || W == 2 || W == 4, "envs of up to 64, 128 or 256 robots");
@@ -434,7 +446,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     int* const ack_l = dyn;
     int* const exlo_l = dyn + n_ul_max * CW;
     int* const exhi_l = dyn + 2 * n_ul_max * CW;
-    int* const hist_l = dyn + (pm.harq_drop ? 3 : 1) * n_ul_max * CW;
+    int* const hist_l = dyn + (WALK ? 0 : (pm.harq_drop ? 3 : 1) * n_ul_max * CW);
     int* const my_hist = hist_l + eloc * 3 * HB;
     // several cells: each gNB's N+I estimate [NC][S] and this slot's interference [NC][S] of this lane's env
     float* const s_ni = reinterpret_cast<float*>(hist_l + envs_pw * 3 * HB) + eloc * 2 * NCS;
@@ -498,6 +510,9 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     olla = ldo(lk.olla, o_r); avg = ldo(lk.avg, o_r);
     qlen = qlen < 0 ? 0 : (qlen > F ? F : qlen);
     if (!act) { sent = 0; floor_ = 0; bsr = 0; sr_t = -1; last_tx = -1; enq = 0; qlen = 0; olla = 0.f; avg = 100.f; }
+    int w_end = 0, w_fin = FIN_NONE;                   // WALK: the queue's first frame
+    uint32_t w_meta = 0u;
+    if constexpr (WALK) { w_end = ldo(lk.q_end, o_fr0); w_fin = ldo(lk.q_fin, o_fr0); w_meta = ldo(lk.q_meta, o_fr0); }
     const uint32_t o_hr0 = (uint32_t)(ee * NCS * R + rr0) * 4u;   // [E][NC S][R] at q = 0
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -619,6 +634,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     if (arr.discard_pdcp && qlen > 0 && (int)T - ldo(lk.q_cap, o_fr0) >= pm.timeout) adm = false;
                     if (adm && qlen < F && size > 0.0f) {
                         const int fr = qlen * R;
+                        if (WALK && qlen == 0) { w_end = enq + nb; w_fin = FIN_NONE; w_meta = 0u; }
                         sto(lk.q_cap + fr, o_fr0, (int)T); sto(lk.q_start + fr, o_fr0, enq);
                         sto(lk.q_end + fr, o_fr0, enq + nb); sto(lk.q_fin + fr, o_fr0, (int)FIN_NONE);
                         sto(lk.q_meta + fr, o_fr0, (uint32_t)(c + 1) << 8); sto(st.q_hid + fr, o_fr0, 0);
@@ -630,6 +646,25 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             }
             if (arr.accepted) sto(arr.accepted, o_r, n_acc);
         }
+    }
+    // the first frame neither completed nor lost, and the one after it
+    int w_f = 0, w_next = 0x7fffffff;
+    uint32_t w_nmeta = 0u;
+    auto walk_fetch = [&](int f) {
+        if (f < qlen) { w_next = ldo(lk.q_end + f * R, o_fr0); w_nmeta = ldo(lk.q_meta + f * R, o_fr0); }
+    };
+    if constexpr (WALK) {
+        if (qlen == 0 || w_fin != FIN_NONE || (w_meta & 1u)) {
+            w_end = 0x7fffffff;
+            for (w_f = 1; w_f < qlen; ++w_f) {
+                const int fr = w_f * R;
+                if (ldo(lk.q_fin + fr, o_fr0) == FIN_NONE && !(ldo(lk.q_meta + fr, o_fr0) & 1u)) {
+                    w_end = ldo(lk.q_end + fr, o_fr0);
+                    break;
+                }
+            }
+        }
+        walk_fetch(w_f + 1);
     }
     // several cells: association of this robot, the N+I estimates of its env (LDS), the env's interference statistic
     int serv = 0, a3_cand = -1, a3_cnt = 0, ho_end = 0, n_ho = 0;
@@ -2101,7 +2136,19 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         }
         }
         // ---- RLC in-order pointer of this slot ----
-        if constexpr (DL) {
+        if constexpr (WALK) {
+            if (any_tx || !ack_known) ack_cur = ack_ptr();
+            ack_known = true;
+            if (__ballot(ack_cur >= w_end) != 0ull) {
+                while (ack_cur >= w_end) {
+                    sto(lv.q_fin + w_f * R, o_fr0, g);
+                    ++w_f;
+                    while (w_f < qlen && (w_nmeta & 1u)) { ++w_f; walk_fetch(w_f); }
+                    w_end = w_f < qlen ? w_next : 0x7fffffff;
+                    walk_fetch(w_f + 1);
+                }
+            }
+        } else if constexpr (DL) {
             // the DL link resolves its frames as the pointer moves (no per-slot history in LDS): under RLC UM the
             // frames an exhausted TB overlaps are lost (mac.py:474-477), then the frames the in-order pointer has
             // passed complete at this slot (mac.py:500-503). Frames before nf are lost or completed, and no
@@ -2140,7 +2187,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
         ++n_ul;
         INET_PH(8);                                // HARQ / OLLA / PF update, counters, in-order pointer
     }
-    const int n_hist = DL ? 0 : (n_ul < n_ul_max ? n_ul : n_ul_max);
+    const int n_hist = DL || WALK ? 0 : (n_ul < n_ul_max ? n_ul : n_ul_max);
 
     // ================================================================ end of step (NRNet._finish)
     {
@@ -2469,7 +2516,7 @@ struct StepArgs {
     InetNrOutputs out;
     int rb;
     unsigned grid;
-    size_t lds;
+    size_t lds, lds_walk;             // dynamic LDS, with and without the per-slot history (WALK builds: without)
     hipStream_t stream;
 };
 typedef void (*StepFn)(const StepArgs&);
@@ -2490,10 +2537,10 @@ template <int S, int P, bool IR, bool VREF, int RBT, int FX = 0>
 void launch_step(const StepArgs& a) {
     if (a.dl)
         hipLaunchKernelGGL((nr_step_kernel<S, P, IR, VREF, RBT, InetNrDlState, 1, FX>), dim3(a.grid),
-                           dim3(STEP_WAVE), a.lds, a.stream, kern_args<InetNrDlState>(a));
+                           dim3(STEP_WAVE), (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrDlState>(a));
     else
         hipLaunchKernelGGL((nr_step_kernel<S, P, IR, VREF, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(STEP_WAVE),
-                           a.lds, a.stream, kern_args<InetNrState>(a));
+                           (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrState>(a));
 }
 
 // the build that fixes these parameters at compile time: 2 (no Rician phasor), 1 (a fixed Rician K), 0 for none
@@ -2513,10 +2560,10 @@ void launch_step_w2(const StepArgs& a) {
     if constexpr (RBT == 128)
         if (a.dl) {
             hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrDlState, 1, FX>), dim3(a.grid), dim3(RBT),
-                               a.lds, a.stream, kern_args<InetNrDlState>(a));
+                               (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrDlState>(a));
             return;
         }
-    hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(RBT), a.lds,
+    hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(RBT), (step_walks(1, FX) ? a.lds_walk : a.lds),
                        a.stream, kern_args<InetNrState>(a));
 }
 
