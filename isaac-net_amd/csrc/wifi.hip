@@ -9,7 +9,7 @@
 // an aligned segment, and a wave holds G envs (G RB <= 64; a launch parameter: fewer envs per wave give more waves,
 // which hides the latency of the serial sub-step chain). The AP's background station is segment-uniform: every lane
 // of the env computes it. The mean-field sums over the stations of the domain (meanfield.SingleView.sum) run over
-// an LDS row in torch's CPU summation order (aten_row_sum), so that only the transcendental functions differ from
+// an LDS row in torch's CPU summation order (row_sum.h), so that only the transcendental functions differ from
 // the CPU path; those are evaluated in double precision and rounded once. The FIFO of each robot lives in LDS
 // columns during the step ([F][64] floats).
 //
@@ -21,10 +21,16 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/inet_wifi.h"
 #include "inet_nr_dev.h"
+#include "row_sum.h"
 
 using namespace inet;
+
+// the row sums' helpers stay inline at every call (a call passes their registers through scratch memory)
+#define ROW_INLINE __attribute__((always_inline))
 
 namespace {
 
@@ -282,30 +288,38 @@ DEV void submit_calls(const InetWifiState& st, int E, const uint8_t* __restrict_
 // offset of R (measured: the general count costs a fifth of the one-AP step through register allocation).
 // CNT: the launch enqueues pm.step_counts first (a build of its own, so that the step without it keeps its register
 // allocation). ZN: AIFS zones (pm.Z > 1; with MA, every station in a lane of its own).
-template <bool DCF, bool MA = false, bool CNT = false, bool ZN = false>
+// BGL: every background station has a lane of its own (R + A <= 64); without, every lane evaluates one beside its robot.
+template <bool DCF, bool MA = false, bool CNT = false, bool ZN = false, bool BGL = true>
 __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetWifiParams pm,
                                                          const int64_t* __restrict__ tin, int input_kind,
                                                          const float* __restrict__ xin,
                                                          const int64_t* __restrict__ hid_in, InetWifiOutputs out,
                                                          int rb, InetDcfState ds, InetDcfParams dp) {
     extern __shared__ float dyn[];
-    __shared__ __align__(16) float s_red[WAVE];
-    __shared__ __align__(16) float s_red4[DCF ? 1 : 3 * WAVE];          // three more rows of station values (dom_sum4)
+    __shared__ __align__(32) float s_red[WAVE];
+    __shared__ __align__(32) float s_red4[DCF ? 1 : 3 * WAVE];          // three more rows of station values (dom_sum4)
     __shared__ uint8_t s_hid0[CNT ? WAVE : 1];            // per env: the enqueue's calls clear the last hazard id
-    __shared__ int s_cmax[CNT ? INET_WIFI_MAX_CLS : 1];   // the largest count of every class (workgroup 0)
+    __shared__ int s_cmax[CNT ? INET_WIFI_MAX_CLS : 1];   // the largest count of every class (the first workgroup)
     __shared__ uint8_t s_dom[MA ? WAVE : 1];              // APs on several channels: each station's domain
     __shared__ float s_rxa[ZN ? WAVE * INET_WIFI_MAX_A : 1];   // hidden nodes: every robot's power at every AP
     __shared__ float s_pos[ZN ? 2 * WAVE : 1];                  // hidden nodes: every robot's position
     const int R = pm.R, F = pm.F, K = pm.K, L = pm.L, G = pm.envs_per_wave;
-    float* s_rem = dyn;                                   // [F][64] bytes left of every frame slot
-    float* s_fin = dyn + F * WAVE;                        // [F][64] finish time, then the compaction staging row
-    uint8_t* s_cls = (uint8_t*)(dyn + 2 * F * WAVE);      // [F][64] class of every frame slot
+    const int F8 = (F + 7) & ~7;
+    float* s_rem = dyn;                                   // [F8][64] bytes left of every frame slot, zeros past slot F
+    float* s_fin = s_rem + F8 * WAVE;                     // [F][64] finish time, then the compaction staging row
+    uint8_t* s_cls = (uint8_t*)(s_fin + F * WAVE);        // [F][64] class of every frame slot
     uint8_t* s_src = s_cls + F * WAVE;                    // [F][64] source slot of every compacted slot
     int32_t* s_stage = (int32_t*)s_fin;
 
+    // the enqueue's global calls are counted by a workgroup of their own, the first (a one-wave pass over every count,
+    // beside the others' steps: behind a step it lengthened the whole launch)
+    if (CNT && blockIdx.x == 0) {
+        submit_calls(st, pm.E, pm.step_counts, (size_t)pm.E * R * pm.step_n_cls, pm.step_n_cls, s_cmax, false);
+        return;
+    }
     const int lane = threadIdx.x;
     const int g = lane / rb, r = lane - g * rb;
-    const int e = blockIdx.x * G + g;
+    const int e = ((int)blockIdx.x - (CNT ? 1 : 0)) * G + g;
     const bool env_ok = g < G && e < pm.E;
     const bool rob = env_ok && r < R;
     const int ec = env_ok ? e : 0, rc = rob ? r : 0;
@@ -378,12 +392,27 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
 
     // ---------------- state ----------------
     int qlen = rob ? st.qlen[ir] : 0;
-    for (int f = 0; f < F; ++f) {
-        const int o = f * WAVE + lane;
-        s_rem[o] = rob && f < qlen ? st.rem[fo + (size_t)f * R] : 0.f;
-        s_cls[o] = rob ? (uint8_t)st.cls[fo + (size_t)f * R] : 0;
-        s_fin[o] = INFINITY;
+    // (a column's words are loaded eight at a time, from the lane's robot or, in idle lanes, from the first: loads under a
+    // condition of their own wait for each other)
+    for (int f0 = 0; f0 < F; f0 += 8) {
+        float rv[8];
+        int cv[8];
+#pragma unroll
+        for (int l = 0; l < 8; ++l) {
+            const size_t q = fo + (size_t)(f0 + l < F ? f0 + l : F - 1) * R;
+            rv[l] = st.rem[q];
+            cv[l] = st.cls[q];
+        }
+#pragma unroll
+        for (int l = 0; l < 8; ++l)
+            if (f0 + l < F) {
+                const int o = (f0 + l) * WAVE + lane;
+                s_rem[o] = rob && f0 + l < qlen ? rv[l] : 0.f;
+                s_cls[o] = rob ? (uint8_t)cv[l] : 0;
+                s_fin[o] = INFINITY;
+            }
     }
+    for (int f = F; f < F8; ++f) s_rem[f * WAVE + lane] = 0.f;
     // counter-RNG keys of this step: the step counter advances before the draws (LevelNet._advance)
     const int ctr = env_ok ? st.ctr_step[ec] + 1 : 0;
     uint32_t hkey = 0;
@@ -398,21 +427,18 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
     int ac = pm.cls_ac[1];
     float capB = cap_bytes(pm, rate, pm.ac_txop[ac]);
     float o_acc = NAN, o_pf = NAN, o_busy = 0.0f;       // wifi_access_ms, wifi_p_fail, wifi_busy
-    // (the row sums read LDS: aten_row_sum_u issues every read before the first add)
-    auto fifo_sum = [&]() -> float {
-        auto xf = [&](int f) { return s_rem[f * WAVE + lane]; };
-        if (F == 16) return aten_row_sum_u<16>(16, xf);
-        if (F <= 16) return aten_row_sum_u<16>(F, xf);
-        if (F <= 32) return aten_row_sum_u<32>(F, xf);
-        if (F <= 64) return aten_row_sum_u<64>(F, xf);
-        return aten_row_sum(F, xf);
+    auto fifo_sum = [&]() ROW_INLINE -> float {
+        return aten_sum_padded(F, [&](int f) ROW_INLINE { return s_rem[f * WAVE + lane]; }, [&](int b) ROW_INLINE {
+            const float* c = s_rem + 8 * b * WAVE + lane;
+            return Row8{c[0], c[WAVE], c[2 * WAVE], c[3 * WAVE], c[4 * WAVE], c[5 * WAVE], c[6 * WAVE], c[7 * WAVE]};
+        });
     };
     if constexpr (!DCF) {
     // The APs' background stations are stations R .. R + A - 1 of the domain (identical: the same weight, window,
     // times and start, so the same tau). With lanes to spare in the segment (rb >= R + A) each runs in its lane like
     // a robot (nothing else), else every lane evaluates one and the sums count it A times.
     const int NS = R + A;                                  // stations of the domain: robots, one per AP
-    const bool bgl = rb >= NS;
+    constexpr bool bgl = BGL;
     const bool is_bg = bgl && env_ok && r >= R && r < NS;
     // APs on several channels (MA builds): one collision domain per channel. A robot is in its serving AP's channel,
     // an AP's background station in the AP's (each has its own lane: R + A <= 64, checked by the entry points).
@@ -464,66 +490,38 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
     const TauW twb = tau_weights(W0b, Wmb);
 
     // sum over the R + A stations of the env (robots in lane order, then the APs' background stations, which all hold
-    // the same values: lane R's, or vb without a spare lane), torch's CPU order. (dom_sum and dom_sum4 each keep
-    // their own copy of the row sum: one shared helper made the compiler spill to scratch.)
-    auto dom_sum = [&](float v, float vb) -> float {
-        __syncthreads();
-        s_red[lane] = v;
-        __syncthreads();
-        const float* row = s_red + gseg * rb;
+    // the same values: lane R's on, or vb without spare lanes), torch's CPU order. The row is the env's segment of an
+    // LDS row: aligned to its rb floats, zeros in the lanes past the last station.
+    auto row_in = [&](float v, float vb) ROW_INLINE -> float { return bgl ? (r < NS ? v : 0.0f) : (r < R ? v : vb); };
+    auto row_sum = [&](const float* base, float vb) ROW_INLINE -> float {
+        const float* row = base + gseg * rb;
         if (hid) return mask_seq_sum(row, vmask, NS);
         if (doms) return dom_seq_sum(row, s_dom + gseg * rb, NS, mydom);
-        if (NS == 17 && bgl) {          // (a 32-lane segment: the row is 128-byte aligned, read 16 bytes at a time)
-            float v[17];
-            const float4* r4 = reinterpret_cast<const float4*>(row);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const float4 q = r4[k];
-                v[4 * k] = q.x; v[4 * k + 1] = q.y; v[4 * k + 2] = q.z; v[4 * k + 3] = q.w;
-            }
-            v[16] = row[16];
-            return aten_row_sum_u<17>(17, [&](int i) { return v[i]; });
-        }
-        auto xr = [&](int i) { return (i < R || bgl) ? row[i] : vb; };
-        if (NS == 17) return aten_row_sum_u<17>(17, xr);
-        if (NS <= 8) return aten_row_sum_u<8>(NS, xr);
-        if (NS <= 16) return aten_row_sum_u<16>(NS, xr);
-        if (NS <= 33) return aten_row_sum_u<33>(NS, xr);
-        return aten_row_sum_u<65>(NS, xr);                  // (R + A <= 65: checked by the entry points)
+        return aten_sum_padded(NS, [&](int i) ROW_INLINE { return row[i]; }, [&](int b) ROW_INLINE {
+            if (!bgl && b == 8) return Row8{vb};            // (station 64 of 65 is a background station)
+            return reinterpret_cast<const Row8*>(row)[b];
+        });
+    };
+    auto dom_sum = [&](float v, float vb) ROW_INLINE -> float {
+        __syncthreads();
+        s_red[lane] = row_in(v, vb);
+        __syncthreads();
+        return row_sum(s_red, vb);
     };
 
     // four such sums at once (one LDS round trip): rows s_red and s_red4[0..2]
     auto dom_sum4 = [&](float v0, float b0, float v1, float b1, float v2, float b2, float v3, float b3, float& o0,
-                        float& o1, float& o2, float& o3) {
+                        float& o1, float& o2, float& o3) ROW_INLINE {
         __syncthreads();
-        s_red[lane] = v0; s_red4[lane] = v1; s_red4[WAVE + lane] = v2; s_red4[2 * WAVE + lane] = v3;
+        s_red[lane] = row_in(v0, b0);
+        s_red4[lane] = row_in(v1, b1);
+        s_red4[WAVE + lane] = row_in(v2, b2);
+        s_red4[2 * WAVE + lane] = row_in(v3, b3);
         __syncthreads();
-        auto sum_row = [&](const float* base, float vb) -> float {
-            const float* row = base + gseg * rb;
-            if (hid) return mask_seq_sum(row, vmask, NS);
-            if (doms) return dom_seq_sum(row, s_dom + gseg * rb, NS, mydom);
-            if (NS == 17 && bgl) {          // (a 32-lane segment: the row is 128-byte aligned, read 16 bytes at a time)
-                float v[17];
-                const float4* r4 = reinterpret_cast<const float4*>(row);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float4 q = r4[k];
-                    v[4 * k] = q.x; v[4 * k + 1] = q.y; v[4 * k + 2] = q.z; v[4 * k + 3] = q.w;
-                }
-                v[16] = row[16];
-                return aten_row_sum_u<17>(17, [&](int i) { return v[i]; });
-            }
-            auto xr = [&](int i) { return (i < R || bgl) ? row[i] : vb; };
-            if (NS == 17) return aten_row_sum_u<17>(17, xr);
-            if (NS <= 8) return aten_row_sum_u<8>(NS, xr);
-            if (NS <= 16) return aten_row_sum_u<16>(NS, xr);
-            if (NS <= 33) return aten_row_sum_u<33>(NS, xr);
-            return aten_row_sum_u<65>(NS, xr);
-        };
-        o0 = sum_row(s_red, b0);
-        o1 = sum_row(s_red4, b1);
-        o2 = sum_row(s_red4 + WAVE, b2);
-        o3 = sum_row(s_red4 + 2 * WAVE, b3);
+        o0 = row_sum(s_red, b0);
+        o1 = row_sum(s_red4, b1);
+        o2 = row_sum(s_red4 + WAVE, b2);
+        o3 = row_sum(s_red4 + 2 * WAVE, b3);
     };
 
     // the smallest value over the stations of this lane's domain (SingleView.min / DomainView.min, meanfield.py:71-73,
@@ -915,66 +913,126 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
     bool det_hit = false;
     uint64_t vmask = 0, dmask = 0;                         // slots still queued after the step; their det flags
     const size_t oo = ir * F;                              // [E][R][F] outputs
-    for (int f = 0; f < F; ++f) {
-        const int o = f * WAVE + lane;
-        int cap = -1;
-        bool dt = false;
-        int hid = 0;
-        if (rob) { cap = st.cap[fo + (size_t)f * R]; dt = st.det[fo + (size_t)f * R] != 0; hid = st.hid[fo + (size_t)f * R]; }
-        const float fin = s_fin[o];
-        const bool dlv = cap >= 0 && fin != INFINITY && fin == fin;
-        const bool timed = cap >= 0 && !dlv && ((t + 1 - (int64_t)cap) >= pm.timeout);
-        newest = dlv && cap > newest ? cap : newest;
-        det_hit = det_hit || (dlv && dt && (int64_t)hid == chid);
-        if (rob) {
-            out.delivered[oo + f] = dlv;
-            out.timed_out[oo + f] = timed;
-            out.cap[oo + f] = cap;
-            out.cls[oo + f] = s_cls[o];
-            out.delay[oo + f] = dlv ? fin - (float)cap : NAN;
+    // (the robot's row of a frame output is contiguous: whole blocks of 8 slots go out in 16-byte stores)
+    const bool vec = (F & 7) == 0 && (((uintptr_t)out.delivered | (uintptr_t)out.timed_out) & 7u) == 0u &&
+                     (((uintptr_t)out.cap | (uintptr_t)out.cls | (uintptr_t)out.delay) & 15u) == 0u;
+    for (int f0 = 0; f0 < F; f0 += 8) {
+        int cp[8], hd[8];
+        uint8_t db[8];
+        float dl[8];
+        uint32_t m_dlv = 0, m_tmo = 0;
+#pragma unroll
+        for (int l = 0; l < 8; ++l) {
+            const size_t q = fo + (size_t)(f0 + l < F ? f0 + l : F - 1) * R;
+            cp[l] = st.cap[q];
+            db[l] = st.det[q];
+            hd[l] = st.hid[q];
         }
-        const bool gone = dlv || timed;
-        if (gone) s_rem[o] = 0.0f;
-        if (!gone && cap >= 0) vmask |= 1ull << f;
-        if (dt && !gone) dmask |= 1ull << f;
-        s_stage[o] = gone ? -1 : cap;                      // the new cap row, staged for the permutation
+#pragma unroll
+        for (int l = 0; l < 8; ++l)
+            if (f0 + l < F) {
+                const int f = f0 + l, o = f * WAVE + lane;
+                const int cap = rob ? cp[l] : -1;
+                const bool dt = rob && db[l] != 0;
+                const float fin = s_fin[o];
+                const bool dlv = cap >= 0 && fin != INFINITY && fin == fin;
+                const bool timed = cap >= 0 && !dlv && ((t + 1 - (int64_t)cap) >= pm.timeout);
+                newest = dlv && cap > newest ? cap : newest;
+                det_hit = det_hit || (dlv && dt && (int64_t)hd[l] == chid);
+                m_dlv |= dlv ? 1u << l : 0u;
+                m_tmo |= timed ? 1u << l : 0u;
+                dl[l] = dlv ? fin - (float)cap : NAN;
+                const bool gone = dlv || timed;
+                if (gone) s_rem[o] = 0.0f;
+                if (!gone && cap >= 0) vmask |= 1ull << f;
+                if (dt && !gone) dmask |= 1ull << f;
+                s_stage[o] = gone ? -1 : cap;              // the new cap row, staged for the permutation
+            }
+        if (!rob) continue;
+        if (vec) {
+            // bit l of the masks to byte l
+            auto bytes = [](uint32_t m) -> uint32_t { return ((m & 0xfu) * 0x204081u) & 0x01010101u; };
+            uint64_t* const od = reinterpret_cast<uint64_t*>(out.delivered + oo + f0);
+            uint64_t* const ot = reinterpret_cast<uint64_t*>(out.timed_out + oo + f0);
+            *od = (uint64_t)bytes(m_dlv) | (uint64_t)bytes(m_dlv >> 4) << 32;
+            *ot = (uint64_t)bytes(m_tmo) | (uint64_t)bytes(m_tmo >> 4) << 32;
+            longlong2* const oc = reinterpret_cast<longlong2*>(out.cap + oo + f0);
+            longlong2* const ok = reinterpret_cast<longlong2*>(out.cls + oo + f0);
+            float4* const oy = reinterpret_cast<float4*>(out.delay + oo + f0);
+#pragma unroll
+            for (int l = 0; l < 8; l += 2) {
+                oc[l >> 1] = make_longlong2(cp[l], cp[l + 1]);
+                ok[l >> 1] = make_longlong2(s_cls[(f0 + l) * WAVE + lane], s_cls[(f0 + l + 1) * WAVE + lane]);
+            }
+            oy[0] = make_float4(dl[0], dl[1], dl[2], dl[3]);
+            oy[1] = make_float4(dl[4], dl[5], dl[6], dl[7]);
+        } else {
+#pragma unroll
+            for (int l = 0; l < 8; ++l)
+                if (f0 + l < F) {
+                    const size_t q = oo + f0 + l;
+                    out.delivered[q] = (m_dlv >> l) & 1u;
+                    out.timed_out[q] = (m_tmo >> l) & 1u;
+                    out.cap[q] = cp[l];
+                    out.cls[q] = s_cls[(f0 + l) * WAVE + lane];
+                    out.delay[q] = dl[l];
+                }
+        }
     }
-    // stable partition (finish_body's cumsum scatter): the queued slots in order, then the others in order
+    // stable partition (finish_body's cumsum scatter): the queued slots in order, then the others in order. Where the
+    // queued slots are the first ones already (every frame of the robot delivered, or none of them), nothing moves, and
+    // the words that only move stay where they are.
     const int nvalid = __builtin_popcountll(vmask);
-    {
+    const bool moves = rob && (vmask & (vmask + 1)) != 0ull;
+    if (__ballot(moves) == 0ull) {
+        if (rob)
+            for (int f = 0; f < F; ++f) {
+                st.cap[fo + (size_t)f * R] = s_stage[f * WAVE + lane];
+                st.det[fo + (size_t)f * R] = (uint8_t)((dmask >> f) & 1ull);
+                st.rem[fo + (size_t)f * R] = s_rem[f * WAVE + lane];
+            }
+    } else if (rob) {
         int gv = 0, gi = nvalid;
         for (int f = 0; f < F; ++f) {
             const int dst = ((vmask >> f) & 1ull) ? gv++ : gi++;
             s_src[dst * WAVE + lane] = (uint8_t)f;
         }
-    }
-    if (rob) {
         // cap (staged above), then every other field through the staging row
-        for (int gdst = 0; gdst < F; ++gdst) st.cap[fo + (size_t)gdst * R] = s_stage[s_src[gdst * WAVE + lane] * WAVE + lane];
-        for (int f = 0; f < F; ++f) {
-            const int o = f * WAVE + lane;
-            s_stage[o] = s_cls[o];
-        }
-        for (int gdst = 0; gdst < F; ++gdst) st.cls[fo + (size_t)gdst * R] = s_stage[s_src[gdst * WAVE + lane] * WAVE + lane];
         for (int gdst = 0; gdst < F; ++gdst) {
             const int sf = s_src[gdst * WAVE + lane];
+            st.cap[fo + (size_t)gdst * R] = s_stage[sf * WAVE + lane];
             st.det[fo + (size_t)gdst * R] = (uint8_t)((dmask >> sf) & 1ull);
         }
-        for (int f = 0; f < F; ++f) s_stage[f * WAVE + lane] = st.hid[fo + (size_t)f * R];
-        for (int gdst = 0; gdst < F; ++gdst) st.hid[fo + (size_t)gdst * R] = s_stage[s_src[gdst * WAVE + lane] * WAVE + lane];
-        for (int f = 0; f < F; ++f) s_stage[f * WAVE + lane] = st.f_nact[fo + (size_t)f * R];
-        for (int gdst = 0; gdst < F; ++gdst) st.f_nact[fo + (size_t)gdst * R] = s_stage[s_src[gdst * WAVE + lane] * WAVE + lane];
-        for (int f = 0; f < F; ++f) s_stage[f * WAVE + lane] = st.f_own[fo + (size_t)f * R];
-        for (int gdst = 0; gdst < F; ++gdst) st.f_own[fo + (size_t)gdst * R] = s_stage[s_src[gdst * WAVE + lane] * WAVE + lane];
+        auto permute = [&](auto* p) {
+            using T = std::remove_reference_t<decltype(*p)>;
+            T* const s_t = reinterpret_cast<T*>(s_stage);
+            for (int f0 = 0; f0 < F; f0 += 8) {
+                T v[8];
+#pragma unroll
+                for (int l = 0; l < 8; ++l) v[l] = p[fo + (size_t)(f0 + l < F ? f0 + l : F - 1) * R];
+#pragma unroll
+                for (int l = 0; l < 8; ++l)
+                    if (f0 + l < F) s_t[(f0 + l) * WAVE + lane] = v[l];
+            }
+            for (int gdst = 0; gdst < F; ++gdst)
+                p[fo + (size_t)gdst * R] = s_t[s_src[gdst * WAVE + lane] * WAVE + lane];
+        };
+        if (moves) {
+            permute(st.cls);
+            permute(st.hid);
+            permute(st.f_nact);
+            permute(st.f_own);
+            permute(st.f_snr);
+        }
         float* s_stf = (float*)s_stage;
-        for (int f = 0; f < F; ++f) s_stf[f * WAVE + lane] = st.f_snr[fo + (size_t)f * R];
-        for (int gdst = 0; gdst < F; ++gdst) st.f_snr[fo + (size_t)gdst * R] = s_stf[s_src[gdst * WAVE + lane] * WAVE + lane];
         for (int f = 0; f < F; ++f) s_stf[f * WAVE + lane] = s_rem[f * WAVE + lane];
         for (int gdst = 0; gdst < F; ++gdst) {
             const float v = s_stf[s_src[gdst * WAVE + lane] * WAVE + lane];
             st.rem[fo + (size_t)gdst * R] = v;
             s_rem[gdst * WAVE + lane] = v;
         }
+    }
+    if (rob) {
         st.qlen[ir] = nvalid;
         out.newest[ir] = newest;
         out.queue_len[ir] = nvalid;
@@ -989,9 +1047,6 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
         st.ctr_step[ec] = ctr;
         st.pending[ec] = 0;
     }
-    // the enqueue's global calls, counted by workgroup 0 at its end (a one-wave pass over every count)
-    if (CNT && blockIdx.x == 0)
-        submit_calls(st, pm.E, pm.step_counts, (size_t)pm.E * R * pm.step_n_cls, pm.step_n_cls, s_cmax, false);
 }
 
 // ======================================================================================= submit kernel
@@ -1133,6 +1188,9 @@ int check_params(const InetWifiParams& p) {
     return INET_WIFI_OK;
 }
 
+// LDS of the step's FIFO columns: bytes left (whole blocks of 8 slots), finish time, class and source of every slot
+size_t step_lds(int F) { return (size_t)WAVE * (4 * ((F + 7) & ~7) + (4 + 1 + 1) * F); }
+
 // the step's enqueue (step_counts): its class count
 int check_step_counts(const InetWifiParams& p) {
     if (p.step_counts && (p.step_n_cls <= 0 || p.step_n_cls > p.n_cls)) return INET_WIFI_EINVAL;
@@ -1159,13 +1217,19 @@ int32_t inet_wifi_step(const InetWifiState* st, const InetWifiParams* prm, const
     InetWifiParams pm = p;
     pm.envs_per_wave = p.envs_per_wave * next_pow2(p.R) / rb > 0 ? p.envs_per_wave * next_pow2(p.R) / rb : 1;
     const int G = pm.envs_per_wave;
-    const unsigned grid = (unsigned)((p.E + G - 1) / G);
+    const unsigned grid = (unsigned)((p.E + G - 1) / G) + (p.step_counts ? 1u : 0u);
     if ((rc = check_step_counts(p))) return rc;
-    const size_t lds = (size_t)p.F * WAVE * (4 + 4 + 1 + 1);
-    auto k = (p.Z > 1 || p.hidden) ? (p.step_counts ? wifi_step_kernel<false, true, true, true>
-                                      : wifi_step_kernel<false, true, false, true>)
-           : p.A > 1 ? (p.step_counts ? wifi_step_kernel<false, true, true> : wifi_step_kernel<false, true, false>)
-                     : (p.step_counts ? wifi_step_kernel<false, false, true> : wifi_step_kernel<false, false, false>);
+    const size_t lds = step_lds(p.F);
+    const bool cnt = p.step_counts != nullptr;
+    auto k = (p.Z > 1 || p.hidden) ? (cnt ? wifi_step_kernel<false, true, true, true>
+                                          : wifi_step_kernel<false, true, false, true>)
+           : p.R + p.A > WAVE      // (65 stations)
+               ? (p.A > 1 ? (cnt ? wifi_step_kernel<false, true, true, false, false>
+                                 : wifi_step_kernel<false, true, false, false, false>)
+                          : (cnt ? wifi_step_kernel<false, false, true, false, false>
+                                 : wifi_step_kernel<false, false, false, false, false>))
+               : (p.A > 1 ? (cnt ? wifi_step_kernel<false, true, true> : wifi_step_kernel<false, true, false>)
+                          : (cnt ? wifi_step_kernel<false, false, true> : wifi_step_kernel<false, false, false>));
     hipLaunchKernelGGL(k, dim3(grid), dim3(WAVE), lds, (hipStream_t)stream, *st, pm, t, input_kind, x, cur_hid, *out,
                        rb, InetDcfState{}, InetDcfParams{});
     return hipGetLastError() == hipSuccess ? INET_WIFI_OK : INET_WIFI_ELAUNCH;
@@ -1217,9 +1281,9 @@ int32_t inet_wifi_dcf_step(const InetWifiState* st, const InetDcfState* ds, cons
     if (input_kind == 0 && p.n_fields < 1) return INET_WIFI_EINVAL;
     const int rb = next_pow2(p.R);
     const int G = p.envs_per_wave;
-    const unsigned grid = (unsigned)((p.E + G - 1) / G);
+    const unsigned grid = (unsigned)((p.E + G - 1) / G) + (p.step_counts ? 1u : 0u);
     if ((rc = check_step_counts(p))) return rc;
-    const size_t lds = (size_t)p.F * WAVE * (4 + 4 + 1 + 1);
+    const size_t lds = step_lds(p.F);
     auto k = p.step_counts ? wifi_step_kernel<true, false, true> : wifi_step_kernel<true, false, false>;
     hipLaunchKernelGGL(k, dim3(grid), dim3(WAVE), lds, (hipStream_t)stream, *st, p, t, input_kind, x, cur_hid, *out,
                        rb, *ds, *dp);
