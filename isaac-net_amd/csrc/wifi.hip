@@ -653,16 +653,36 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
                 }
             p = 1.0f - num / clamp_min(O, 1e-12f);
         };
-        for (int it = 0; it < pm.fp_iters; ++it) {
-            tau = clampf(tau, 1e-7f, 0.999f);
-            if (!bgl) tau_b = clampf(tau_b, 1e-7f, 0.999f);
-            if constexpr (ZN) failz(); else fail();
-            tau = tau + pm.damp * (tau_of_p(p, W0s, Wms, L, tw) - tau);
-            if (!bgl) tau_b = tau_b + pm.damp * (tau_of_p(pb, W0b, Wmb, L, twb) - tau_b);
+        // A sub-step in which no station of the wavefront contends (the queues of a lightly loaded cell are empty for most
+        // of a step): every weight is 0, so the domain sums are 0, the failure probability is 1 - fer1 in every
+        // iteration and only the damped step of tau is left, to the same bits as below.
+        const bool quiet = !ZN && wb == 0.0f && __ballot(act) == 0ull;
+        if (quiet) {
+            ok = pm.fer1;
+            p = pb = 1.0f - ok;
+            const float tp = tau_of_p(p, W0s, Wms, L, tw);
+            const float tpb = bgl ? 0.0f : tau_of_p(pb, W0b, Wmb, L, twb);
+            for (int it = 0; it < pm.fp_iters; ++it) {
+                tau = clampf(tau, 1e-7f, 0.999f);
+                tau = tau + pm.damp * (tp - tau);
+                if (!bgl) {
+                    tau_b = clampf(tau_b, 1e-7f, 0.999f);
+                    tau_b = tau_b + pm.damp * (tpb - tau_b);
+                }
+            }
+        } else {
+            for (int it = 0; it < pm.fp_iters; ++it) {
+                tau = clampf(tau, 1e-7f, 0.999f);
+                if (!bgl) tau_b = clampf(tau_b, 1e-7f, 0.999f);
+                if constexpr (ZN) failz(); else fail();
+                tau = tau + pm.damp * (tau_of_p(p, W0s, Wms, L, tw) - tau);
+                if (!bgl) tau_b = tau_b + pm.damp * (tau_of_p(pb, W0b, Wmb, L, twb) - tau_b);
+            }
         }
         tau = clampf(tau, 1e-7f, 0.999f);
         if (!bgl) tau_b = clampf(tau_b, 1e-7f, 0.999f);
-        if constexpr (ZN) failz(); else fail();
+        if constexpr (ZN) failz();
+        else if (!quiet) fail();
         const float r_o = (ws * tau) / (1.0f - tau), r_b = bgl ? 0.0f : (wb * tau_b) / (1.0f - tau_b);
         const float wt_o = ws * tau, wt_b = wb * tau_b;
         // ---- retry-limit loss inputs (wifi/engine.py:375-381; they need only this sub-step's p, so they are
@@ -690,6 +710,9 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
                     tslot = tslot + piz[z] * ((pm.slot_us * idle + idle * a1) + p_coll * tcav);
                     p_idle = p_idle + piz[z] * idle;
                 }
+        } else if (quiet) {                            // (idle = 1, every sum 0)
+            tslot = pm.slot_us;
+            p_idle = 1.0f;
         } else {
             const float idle = exp_r(S);
             float a0, a1, gd, gg;
@@ -705,15 +728,18 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
         const float lam = mu * pm.dt_us;
         float n_acc, c1 = 0.f;
         if (pm.access_noise == 0) {
-            const float u = uniform_bits(elem_hash(key_acc, (uint32_t)(k * R + rc)));
-            const float ll = log_r(clamp_min(lam, 1e-30f));
-            double cum = 0.0;
+            // (a station that does not contend has lam = 0: the CDF is 1 at once where lgamma(1) = 0)
             int n = 0;
-            for (int kk = 0; kk < pm.n_acc_max; ++kk) {
-                const float lp = ((float)kk * ll - lam) - pm.lgamma[kk];
-                cum += (double)exp_r(lp);
-                if (!(u > (float)cum)) break;      // the CDF never decreases: the count is the first k with u <= CDF
-                ++n;
+            if (act || pm.lgamma[0] != 0.0f) {
+                const float u = uniform_bits(elem_hash(key_acc, (uint32_t)(k * R + rc)));
+                const float ll = log_r(clamp_min(lam, 1e-30f));
+                double cum = 0.0;
+                for (int kk = 0; kk < pm.n_acc_max; ++kk) {
+                    const float lp = ((float)kk * ll - lam) - pm.lgamma[kk];
+                    cum += (double)exp_r(lp);
+                    if (!(u > (float)cum)) break;  // the CDF never decreases: the count is the first k with u <= CDF
+                    ++n;
+                }
             }
             n_acc = (float)n;
         } else {
@@ -747,13 +773,15 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
             }
         };
         {
-            // (the next frame's bytes and class are read before this frame is served)
-            float rm_n = qlen > 0 ? s_rem[lane] : 0.0f;
-            int cl_n = qlen > 0 ? (int)s_cls[lane] : 0;
-            for (int f = 0; f < qlen; ++f) {
+            // (the next frame's bytes and class are read before this frame is served; an empty queue's frames stay as
+            // they are)
+            const int nf = q > 0.0f ? qlen : 0;
+            float rm_n = nf > 0 ? s_rem[lane] : 0.0f;
+            int cl_n = nf > 0 ? (int)s_cls[lane] : 0;
+            for (int f = 0; f < nf; ++f) {
                 const float rm = rm_n;
                 const int c = cl_n;
-                if (f + 1 < qlen) {
+                if (f + 1 < nf) {
                     rm_n = s_rem[(f + 1) * WAVE + lane];
                     cl_n = (int)s_cls[(f + 1) * WAVE + lane];
                 }
