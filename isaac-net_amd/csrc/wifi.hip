@@ -42,16 +42,26 @@ DEV float exp_r(float x) { return (float)exp((double)x); }
 DEV float log_r(float x) { return (float)log((double)x); }
 DEV float log1p_r(float x) { return (float)log1p((double)x); }
 DEV float pow_r(float x, float y) { return (float)pow((double)x, (double)y); }
+// x ** n for an integer 0 <= n <= 4096: pow_count's double-precision binary powering, rounded once
+DEV float pow_i(float x, int n) {
+    double r = 1.0, b = (double)x;
+    while (n) {
+        if (n & 1) r *= b;
+        b *= b;
+        n >>= 1;
+    }
+    return (float)r;
+}
 // x ** n for a Python int exponent n (torch pow with a scalar: 1 copies, 2 and 3 multiply, others pow)
 DEV float pow_int_torch(float x, int n) {
     if (n == 1) return x;
     if (n == 2) return x * x;
     if (n == 3) return (x * x) * x;
-    return pow_count(x, (float)n);
+    return pow_i(x, n);
 }
 // p ** k of tau(p) (torch pow of two float tensors) for an integer k >= 0: double-precision binary powering,
 // rounded once
-DEV float pow_k(float p, int k) { return pow_count(p, (float)k); }
+DEV float pow_k(float p, int k) { return pow_i(p, k); }
 DEV float fminn(float a, float b) { return a != a ? a : (b != b ? b : (a < b ? a : b)); }   // torch.minimum
 
 // AccessTiming.cap_bytes (wifi/phy.py:130-139): application bytes one access carries
@@ -98,8 +108,9 @@ DEV TauW tau_weights(float W0, float Wm) {
     }
     return t;
 }
+template <bool LS>
 DEV float tau_of_p(float p, float W0, float Wm, int L, const TauW& tw) {
-    if (L < 8) {
+    if constexpr (LS) {
         // (unrolled to the 7-stage bound; the stage terms are the running product's, and the four partial sums take
         // stages 0..3 one each and the later ones into the first when L >= 4, every stage into the first below 4)
         const double pd = (double)p;
@@ -125,13 +136,14 @@ DEV float tau_of_p(float p, float W0, float Wm, int L, const TauW& tw) {
                 if (k < L) { n0 += pk[k]; d0 += tk[k]; }
         }
         return (((n0 + n1) + n2) + n3) / (((d0 + d1) + d2) + d3);
+    } else {
+        float num = aten_row_sum(L, [&](int k) { return pow_k(p, k); });
+        float den = aten_row_sum(L, [&](int k) {
+            float wk = fminn(W0 * exp2f((float)k), Wm);
+            return pow_k(p, k) * ((wk + 1.0f) * 0.5f);
+        });
+        return num / den;
     }
-    float num = aten_row_sum(L, [&](int k) { return pow_k(p, k); });
-    float den = aten_row_sum(L, [&](int k) {
-        float wk = fminn(W0 * exp2f((float)k), Wm);
-        return pow_k(p, k) * ((wk + 1.0f) * 0.5f);
-    });
-    return num / den;
 }
 
 // U{0..W-1} from an element hash: ((h >> 8) W) >> 24
@@ -288,8 +300,10 @@ DEV void submit_calls(const InetWifiState& st, int E, const uint8_t* __restrict_
 // offset of R (measured: the general count costs a fifth of the one-AP step through register allocation).
 // CNT: the launch enqueues pm.step_counts first (a build of its own, so that the step without it keeps its register
 // allocation). ZN: AIFS zones (pm.Z > 1; with MA, every station in a lane of its own).
+// LS: at most 7 transmission attempts (L < 8; the backoff stages unrolled). With the general stage sums and their powf in
+// the same build its code was 18600 lines, most of it never run, and the registers of both counted.
 // BGL: every background station has a lane of its own (R + A <= 64); without, every lane evaluates one beside its robot.
-template <bool DCF, bool MA = false, bool CNT = false, bool ZN = false, bool BGL = true>
+template <bool DCF, bool MA = false, bool CNT = false, bool ZN = false, bool BGL = true, bool LS = true>
 __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetWifiParams pm,
                                                          const int64_t* __restrict__ tin, int input_kind,
                                                          const float* __restrict__ xin,
@@ -548,6 +562,7 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
 
     float acc_sum = 0.f, acc_n = 0.f, p_sum = 0.f, busy_sum = 0.f;
     const float tf = (float)t;
+    int head = 0;                                          // the frames before it are served
     for (int k = 0; k < K; ++k) {
         const float q = fifo_sum();
         const bool act = rob && q > 0.f && link && roam <= 0;
@@ -660,8 +675,8 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
         if (quiet) {
             ok = pm.fer1;
             p = pb = 1.0f - ok;
-            const float tp = tau_of_p(p, W0s, Wms, L, tw);
-            const float tpb = bgl ? 0.0f : tau_of_p(pb, W0b, Wmb, L, twb);
+            const float tp = tau_of_p<LS>(p, W0s, Wms, L, tw);
+            const float tpb = bgl ? 0.0f : tau_of_p<LS>(pb, W0b, Wmb, L, twb);
             for (int it = 0; it < pm.fp_iters; ++it) {
                 tau = clampf(tau, 1e-7f, 0.999f);
                 tau = tau + pm.damp * (tp - tau);
@@ -675,8 +690,8 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
                 tau = clampf(tau, 1e-7f, 0.999f);
                 if (!bgl) tau_b = clampf(tau_b, 1e-7f, 0.999f);
                 if constexpr (ZN) failz(); else fail();
-                tau = tau + pm.damp * (tau_of_p(p, W0s, Wms, L, tw) - tau);
-                if (!bgl) tau_b = tau_b + pm.damp * (tau_of_p(pb, W0b, Wmb, L, twb) - tau_b);
+                tau = tau + pm.damp * (tau_of_p<LS>(p, W0s, Wms, L, tw) - tau);
+                if (!bgl) tau_b = tau_b + pm.damp * (tau_of_p<LS>(pb, W0b, Wmb, L, twb) - tau_b);
             }
         }
         tau = clampf(tau, 1e-7f, 0.999f);
@@ -749,44 +764,48 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
         const float served = fminn(q, n_acc * B) * w;
 
         // ---- FIFO service, finish times, loss (serve_fifo, wifi/engine.py:361-383)
+        // (one pass takes the bytes off the frames, from the first unserved one, and marks those that finish; their
+        // finish times and losses follow, a finished frame of every lane at a time, wherever in the queues they are:
+        // the divisions and powers within the pass ran once for every slot in which any lane's frame finished)
         double cacc = 0.0;
         float prev_nc = 0.0f;
-        auto serve = [&](int f, float rm, int c) {
-            const int o = f * WAVE + lane;
-            cacc += (double)rm;
-            const float cum = (float)cacc;
-            const float nc = clamp_min(cum - served, 0.0f);
-            const float nw = nc - prev_nc;
-            prev_nc = nc;
-            const bool fin = rm > 0.0f && nw <= 1e-3f;
-            s_rem[o] = fin ? 0.0f : nw;
-            if (fin) {
-                const float j = clamp_min(ceilf(cum / B - 1e-6f), 1.0f);
-                float frac = pm.access_noise == 0 ? j / (n_acc + 1.0f) : (j - credit) / clamp_min(lam, 1e-9f);
-                frac = clampf(frac, 0.0f, 1.0f);
-                const float tfin = fminn(tf + ((float)k + frac) / (float)K, (tf + 1.0f) - 1e-6f);
-                const float size = pm.sizes[(c > 1 ? (c < pm.n_cls ? c : pm.n_cls) : 1) - 1];
-                const float n_frame = clamp_min(ceilf(size / B), 1.0f);
-                const float p_lost = 1.0f - pow_count(1.0f - pbl, n_frame);
-                const float u = uniform_bits(elem_hash(key_loss, (uint32_t)(rc * F + f)));
-                if (!(u < p_lost)) s_fin[o] = tfin;
-            }
-        };
-        {
-            // (the next frame's bytes and class are read before this frame is served; an empty queue's frames stay as
-            // they are)
-            const int nf = q > 0.0f ? qlen : 0;
-            float rm_n = nf > 0 ? s_rem[lane] : 0.0f;
-            int cl_n = nf > 0 ? (int)s_cls[lane] : 0;
-            for (int f = 0; f < nf; ++f) {
-                const float rm = rm_n;
-                const int c = cl_n;
-                if (f + 1 < nf) {
-                    rm_n = s_rem[(f + 1) * WAVE + lane];
-                    cl_n = (int)s_cls[(f + 1) * WAVE + lane];
+        const int nf = q > 0.0f ? qlen : 0;                // (an empty queue's frames stay as they are)
+        uint64_t fins = 0ull;
+        for (int f0 = head; f0 < nf; f0 += 4) {
+            float rm[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) rm[j] = s_rem[(f0 + j < F ? f0 + j : F - 1) * WAVE + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (f0 + j < nf) {
+                    const int f = f0 + j, o = f * WAVE + lane;
+                    cacc += (double)rm[j];
+                    const float cum = (float)cacc;
+                    const float nc = clamp_min(cum - served, 0.0f);
+                    const float nw = nc - prev_nc;
+                    prev_nc = nc;
+                    const bool fin = rm[j] > 0.0f && nw <= 1e-3f;
+                    const float left = fin ? 0.0f : nw;
+                    s_rem[o] = left;
+                    if (fin) {
+                        fins |= 1ull << f;
+                        s_fin[o] = cum;
+                    }
+                    head = f == head && left == 0.0f ? f + 1 : head;
                 }
-                serve(f, rm, c);
-            }
+        }
+        for (; fins; fins &= fins - 1ull) {
+            const int f = __builtin_ctzll(fins), o = f * WAVE + lane, c = (int)s_cls[o];
+            const float cum = s_fin[o];
+            const float j = clamp_min(ceilf(cum / B - 1e-6f), 1.0f);
+            float frac = pm.access_noise == 0 ? j / (n_acc + 1.0f) : (j - credit) / clamp_min(lam, 1e-9f);
+            frac = clampf(frac, 0.0f, 1.0f);
+            const float tfin = fminn(tf + ((float)k + frac) / (float)K, (tf + 1.0f) - 1e-6f);
+            const float size = pm.sizes[(c > 1 ? (c < pm.n_cls ? c : pm.n_cls) : 1) - 1];
+            const float n_frame = clamp_min(ceilf(size / B), 1.0f);
+            const float p_lost = 1.0f - pow_count(1.0f - pbl, n_frame);
+            const float u = uniform_bits(elem_hash(key_loss, (uint32_t)(rc * F + f)));
+            s_fin[o] = u < p_lost ? INFINITY : tfin;
         }
         if (pm.access_noise == 1 && act) credit = fifo_sum() > 0.f ? c1 - n_acc : 0.0f;
         roam = roam - 1 > 0 ? roam - 1 : 0;
@@ -1216,6 +1235,24 @@ int check_params(const InetWifiParams& p) {
     return INET_WIFI_OK;
 }
 
+// the mean-field step's build for these parameters
+template <bool LS>
+auto mf_kernel(const InetWifiParams& p) {
+    const bool cnt = p.step_counts != nullptr;
+    if (p.Z > 1 || p.hidden)
+        return cnt ? wifi_step_kernel<false, true, true, true, true, LS>
+                   : wifi_step_kernel<false, true, false, true, true, LS>;
+    if (p.R + p.A > WAVE)                   // (65 stations)
+        return p.A > 1 ? (cnt ? wifi_step_kernel<false, true, true, false, false, LS>
+                              : wifi_step_kernel<false, true, false, false, false, LS>)
+                       : (cnt ? wifi_step_kernel<false, false, true, false, false, LS>
+                              : wifi_step_kernel<false, false, false, false, false, LS>);
+    return p.A > 1 ? (cnt ? wifi_step_kernel<false, true, true, false, true, LS>
+                          : wifi_step_kernel<false, true, false, false, true, LS>)
+                   : (cnt ? wifi_step_kernel<false, false, true, false, true, LS>
+                          : wifi_step_kernel<false, false, false, false, true, LS>);
+}
+
 // LDS of the step's FIFO columns: bytes left (whole blocks of 8 slots), finish time, class and source of every slot
 size_t step_lds(int F) { return (size_t)WAVE * (4 * ((F + 7) & ~7) + (4 + 1 + 1) * F); }
 
@@ -1248,16 +1285,7 @@ int32_t inet_wifi_step(const InetWifiState* st, const InetWifiParams* prm, const
     const unsigned grid = (unsigned)((p.E + G - 1) / G) + (p.step_counts ? 1u : 0u);
     if ((rc = check_step_counts(p))) return rc;
     const size_t lds = step_lds(p.F);
-    const bool cnt = p.step_counts != nullptr;
-    auto k = (p.Z > 1 || p.hidden) ? (cnt ? wifi_step_kernel<false, true, true, true>
-                                          : wifi_step_kernel<false, true, false, true>)
-           : p.R + p.A > WAVE      // (65 stations)
-               ? (p.A > 1 ? (cnt ? wifi_step_kernel<false, true, true, false, false>
-                                 : wifi_step_kernel<false, true, false, false, false>)
-                          : (cnt ? wifi_step_kernel<false, false, true, false, false>
-                                 : wifi_step_kernel<false, false, false, false, false>))
-               : (p.A > 1 ? (cnt ? wifi_step_kernel<false, true, true> : wifi_step_kernel<false, true, false>)
-                          : (cnt ? wifi_step_kernel<false, false, true> : wifi_step_kernel<false, false, false>));
+    auto k = p.L < 8 ? mf_kernel<true>(p) : mf_kernel<false>(p);
     hipLaunchKernelGGL(k, dim3(grid), dim3(WAVE), lds, (hipStream_t)stream, *st, pm, t, input_kind, x, cur_hid, *out,
                        rb, InetDcfState{}, InetDcfParams{});
     return hipGetLastError() == hipSuccess ? INET_WIFI_OK : INET_WIFI_ELAUNCH;
