@@ -117,10 +117,10 @@ class HipWifiEngine:
         self.reset(None)
 
     # ------------------------------------------------------------------ buffers and constants
-    # wavefronts of a step that the chip holds at once: the mean-field kernel takes one per SIMD (its registers), so one
-    # more starts a second round of the whole serial chain; the per-slot kernel two or more. us per step by envs per
-    # wavefront, mean-field 2048 x 16: 437 (one), 230 (two); 4096 x 6: 1138, 583, 302, 306 (1, 2, 4, 8); 1024 x 16: 223,
-    # 231; per-slot 4096 x 16: 94, 68, 73 (1, 2, 4), 2048 x 30: 70, 73 (1, 2)
+    # wavefronts of a step up to which another one costs next to nothing: the mean-field kernel is one serial chain that
+    # leaves a SIMD little room for a second, the per-slot kernel has more. us per step by envs per wavefront,
+    # mean-field 2048 x 16: 228 (one), 217 (two); 4096 x 16: 378, 243; 4096 x 6: 269, 192, 190, 193 (1, 2, 4, 8);
+    # 1024 x 16: 209, 214; per-slot 4096 x 16: 78, 53, 51 (1, 2, 4), 2048 x 30: 63, 63 (1, 2)
     _waves = 1024
 
     def _auto_envs_per_wave(self, rb):
