@@ -41,7 +41,7 @@
 extern "C" {
 #endif
 
-#define INET_NR_ABI_VERSION 15
+#define INET_NR_ABI_VERSION 16
 #define INET_NR_MAX_S 32          /* subbands (RBGs) */
 #define INET_NR_MAX_P 16          /* HARQ processes */
 #define INET_NR_MAX_R 256         /* robots per env: a segment of one 64-wide wavefront (up to 64), or two / four
@@ -132,7 +132,7 @@ typedef struct InetNrState {
 /* Device tables (PHY) and the host constants that go with them. */
 typedef struct InetNrTables {
     const float *bler;        /* [M][C][G] code-block BLER */
-    const float *thr_ref;     /* [M] target-BLER SINR of one 10-PRB RBG */
+    const float *thr_ref;     /* [M] target-BLER SINR of one 10-PRB RBG; with thr_ext [M + 2] */
     const float *se;          /* [M] spectral efficiency Qm R */
     const float *beta;        /* [M] EESM beta */
     const float *rate;        /* [M] code rate R */
@@ -148,11 +148,11 @@ typedef struct InetNrTables {
     int32_t M, C, G, NPRB, EQW, mcs_max;
     int32_t thr_monotone;     /* informational: thr_ref[0..mcs_max] non-decreasing (the kernels search its suffix
                                  minima, which give the highest passing MCS for any table) */
-    int32_t thr_ext;          /* 1: thr_ref holds two further words a, k: no TB of MCS m meets the BLER target at an
-                                 effective SINR (dB, OLLA offset included) below a + m / k, with a margin for the
-                                 float32 rounding of effective SINRs from -14 dB up, and none meets it below -14 dB;
-                                 the link adaptation starts its search there. 0: it starts at mcs_max. The results
-                                 are the same */
+    int32_t thr_ext;          /* (ABI 16; an unused word before) 1: thr_ref holds two further words a, k: no TB of MCS m
+                                 meets the BLER target at an effective SINR (dB, OLLA offset included) below
+                                 a + m / k, with a margin for the float32 rounding of effective SINRs from -14 dB up,
+                                 and none meets it below -14 dB; the link adaptation starts its search there.
+                                 0: it starts at mcs_max. The results are the same */
 } InetNrTables;
 
 /* Config constants of the step (derived on the host from NRConfig). */

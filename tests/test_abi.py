@@ -2,6 +2,7 @@
 declare, and the ctypes mirrors of the structs have the C layout (checked against sizeof / offsetof from the headers
 compiled by gcc). No compute entry point is called here."""
 import ctypes
+import hashlib
 import os
 import re
 import subprocess
@@ -37,7 +38,7 @@ def test_library_exports_every_declared_symbol():
     for n in names:
         assert hasattr(lib, n), n
     lib.inet_nr_abi_version.restype = ctypes.c_int32
-    assert lib.inet_nr_abi_version() == _lib.ABI_VERSION == 15
+    assert lib.inet_nr_abi_version() == _lib.ABI_VERSION == 16
     lib.inet_nr_build_info.restype = ctypes.c_char_p
     assert b"gfx950" in lib.inet_nr_build_info()
     wifi = declared_functions(WIFI_HEADER, "inet_wifi_")
@@ -83,3 +84,40 @@ def test_load_refuses_missing_library(tmp_path):
             _lib.load(str(tmp_path / "nope.so"))
         finally:
             _lib._LIB = saved
+
+
+# version -> digest of the header's structs without comments: a word that is added, renamed or given another meaning takes
+# a version of its own, so that a caller built against an older header is told so by inet_nr_abi_version. (15 ended
+# InetNrTables with an unused word, which such a caller may leave unset; since 16 it says that thr_ref is longer.)
+STRUCT_DIGESTS = {15: "f9a8729d357584a2", 16: "1411f638cc4326b3"}
+
+
+def struct_digest(src):
+    src = re.sub(r"/\*.*?\*/", " ", src, flags=re.S)
+    structs = re.findall(r"typedef\s+struct\s+\w+\s*\{.*?\}\s*\w+\s*;", src, flags=re.S)
+    assert len(structs) >= 8
+    return hashlib.sha256(" ".join(" ".join(structs).split()).encode()).hexdigest()[:16]
+
+
+def test_struct_words_belong_to_the_version():
+    src = open(HEADER).read()
+    version = int(re.search(r"#define\s+INET_NR_ABI_VERSION\s+(\d+)", src).group(1))
+    assert struct_digest(src) == STRUCT_DIGESTS[version]
+
+
+@pytest.mark.parametrize("nr,wifi", [(-1, 0), (1, 0), (0, -1)])
+def test_load_refuses_another_version(tmp_path, nr, wifi):
+    names = declared_functions() + declared_functions(WIFI_HEADER, "inet_wifi_")
+    ret = {"inet_nr_abi_version": _lib.ABI_VERSION + nr, "inet_wifi_abi_version": _lib.WIFI_ABI_VERSION + wifi}
+    (tmp_path / "old.c").write_text("\n".join(
+        'const char *inet_nr_build_info(void) { return ""; }' if n == "inet_nr_build_info" else
+        f"int {n}(void) {{ return {ret.get(n, 0)}; }}" for n in names))
+    so = str(tmp_path / "libold.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", so, str(tmp_path / "old.c")], check=True)
+    _lib._LIB, saved = None, _lib._LIB
+    try:
+        with pytest.raises(RuntimeError, match="ABI version"):
+            _lib.load(so)
+        assert _lib._LIB is None
+    finally:
+        _lib._LIB = saved
