@@ -150,9 +150,9 @@ typedef struct InetNrTables {
                                  minima, which give the highest passing MCS for any table) */
     int32_t thr_ext;          /* (ABI 16; an unused word before) 1: thr_ref holds two further words a, k: no TB of MCS m
                                  meets the BLER target at an effective SINR (dB, OLLA offset included) below
-                                 a + m / k, with a margin for the float32 rounding of effective SINRs from -14 dB up,
-                                 and none meets it below -14 dB; the link adaptation starts its search there.
-                                 0: it starts at mcs_max. The results are the same */
+                                 a + m / k, with a margin for the effective SINR's float32 rounding before an OLLA
+                                 offset of up to 10 dB, and none meets it below -14 dB; the link adaptation starts its
+                                 search there. 0: it starts at mcs_max. The results are the same */
 } InetNrTables;
 
 /* Config constants of the step (derived on the host from NRConfig). */

@@ -1827,9 +1827,9 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             s_la_f[2 * CW + lane] = eff_md;
             // Where the search starts. The EESM effective SINR of a row is at most its largest held SINR, so no MCS
             // passes whose floor (the SINR that a TB of it needs at the least, PhyTables.la_floor) lies above that
-            // plus the OLLA offset, and the floors lie above the line la_a + m / la_m1, which also takes the
-            // float32 rounding of the log-sum-exp (from -14 dB; below, no MCS passes). Without a bound a robot at the
-            // cell edge walks down the whole table, a few candidates a round: default configuration 256 x 16 488 us
+            // plus the OLLA offset, and the floors lie above the line la_a + m / la_m1, less the float32 rounding of
+            // the log-sum-exp before that offset (no MCS passes below -14 dB). Without a bound a robot at the cell
+            // edge walks down the whole table, a few candidates a round: default configuration 256 x 16 488 us
             // without it, 385 us with it, 1024 x 32 570 and 462, three cells 1024 x 64 692 and 617. A search of the
             // floors themselves from the tighter mean of the linear SINRs measured slower where few robots send (rl
             // 4096 x 32 221 us against 217: LDS reads and a logarithm on the slot's serial chain).

@@ -205,9 +205,10 @@ class PhyTables:
         return np.where(j <= 1, -np.inf, np.where(j >= self.G, np.inf, f))
 
     def la_line(self):
-        """(a, k) float32 with a + m / k below every MCS's floor, less the float32 rounding of an EESM effective SINR:
-        at most 1e-5 beta (linear), in dB at -14 dB or more; None where some MCS has no floor or one below -14 dB, or
-        the floors do not rise."""
+        """(a, k) float32 with a + m / k below every MCS's floor, less the float32 rounding of an EESM effective SINR;
+        None where some MCS has no floor or one below -14 dB, or the floors do not rise. The rounding, at most 1e-5
+        beta (linear: two log-sum-exps under 8, each within 8 units of 2^-21), is there before the OLLA offset of up
+        to 10 dB is added: MCS m passes from f - 10 dB on at the earliest, and there it weighs the most dB."""
         f = self.la_floor()
         ok = np.isfinite(f)
         if ok.sum() < 2 or (f < -13.5).any():
@@ -216,8 +217,8 @@ class PhyTables:
         slope = float(np.polyfit(m, f[ok], 1)[0])
         if slope <= 1e-3:
             return None
-        margin = 10 * math.log10(1 + 1e-5 * float(self.beta.max()) / 10 ** -1.4) + 2e-3
-        return _f32((f[ok] - slope * m).min() - margin), _f32(1 / slope)
+        margin = -10 * np.log10(1.0 - 1e-5 * self.beta[ok] / 10 ** ((f[ok] - 10.0) / 10)) + 2e-3
+        return _f32((f[ok] - slope * m - margin).min()), _f32(1 / slope)
 
     def tbs_all(self, n_prb, nsym, dmrs=12, oh=0):
         """TBS (bits) of every MCS for PRB counts n_prb [...] -> [..., M] int64."""

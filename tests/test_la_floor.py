@@ -38,6 +38,20 @@ def test_no_tb_passes_below_the_floor(table, target, nprb, nsym):
         assert line[0] + m / line[1] < f[m] - 1e-3, m
 
 
+@pytest.mark.parametrize("table", [1, 2])
+@pytest.mark.parametrize("target", [1e-5, 1e-3, 0.01, 0.1, 0.3, 0.5, 0.9, 0.99])
+def test_line_takes_the_rounding_before_the_olla_offset(table, target):
+    """An effective SINR's float32 rounding, at most 1e-5 beta (linear), is there before the OLLA offset of up to 10 dB:
+    the largest SINR that this rounding and that offset can lift to an MCS's floor still lies above the line."""
+    t = P.PhyTables(table, target, 4, None)
+    a, k = t.la_line()
+    f = t.la_floor()
+    for m in range(t.M):
+        if np.isfinite(f[m]):
+            least = 10 * np.log10(10 ** ((f[m] - 10.0) / 10) - 1e-5 * float(t.beta[m])) + 10.0
+            assert float(a) + m / float(k) < least - 1e-3, m
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kw", [dict(), dict(mcs_table=2, ul_mcs_max=20), dict(eff_sinr="mean_db"),
                                 dict(n_prb=273, rbg_size=35), dict(ul_amc_alloc="previous", ul_power="whole_band"),
@@ -66,3 +80,33 @@ def test_search_from_the_floor_equals_the_full_search(kw):
         assert torch.equal(a.st[k].nan_to_num(-7.0) if a.st[k].is_floating_point() else a.st[k],
                            b.st[k].nan_to_num(-7.0) if b.st[k].is_floating_point() else b.st[k]), k
     assert int(a.st["ctr"][:, 0].sum()) > 100
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw", [dict(), dict(mcs_table=2), dict(n_prb=273, bler_target=0.5)])
+def test_search_from_the_floor_at_the_largest_olla_offset(kw):
+    """Robots at OLLA offsets of +10, 9.7 and -9.7 dB with reference SINRs from -28 to -4 dB: the lowest MCS passes at raw
+    SINRs where the rounding of the log-sum-exp weighs the most."""
+    cfg = P.NRConfig(control_step_ms=20.0, msg_sizes=(3000.0,), n_harq=4, seed=0, **kw)
+    E, R, S = 16, 48, cfg.n_subbands
+    print(f"link adaptation at the largest OLLA offset, {kw}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    a, b = (P.make_engine("L2", E, R, DEV, cfg, seed=5) for _ in range(2))
+    b._ctab.thr_ext = 0
+    for s in range(4):
+        off = torch.full((E, R), 10.0, device=DEV)
+        off[:, 1::4], off[:, 2::4] = 9.7, -9.7
+        for e in (a, b):
+            e.st["olla"].copy_(off)
+        # (SNR input is the reference SINR: the power split over the PRBs and the fading come on top)
+        snr = torch.rand(E, R, 1, generator=g, device=DEV) * 24.0 - 28.0
+        snr = (snr + torch.randn(E, R, S, generator=g, device=DEV) * 0.5).contiguous()
+        c = torch.ones(E, R, 1, dtype=torch.uint8, device=DEV)
+        oa, ob = a.step(None, snr_db=snr, arrivals=c), b.step(None, snr_db=snr, arrivals=c)
+        for k in oa:
+            assert torch.equal(oa[k].nan_to_num(-7.0) if oa[k].is_floating_point() else oa[k],
+                               ob[k].nan_to_num(-7.0) if ob[k].is_floating_point() else ob[k]), (s, k)
+        for k in ("h_meta", "h_tbs", "sent", "csi", "olla", "ctr"):
+            assert torch.equal(a.st[k], b.st[k]), (s, k)
+    mcs = (a.st["h_meta"] >> 16) & 0xff
+    assert int(a.st["ctr"][:, 0].sum()) > 50 and int((mcs == 0).sum()) > 0 and int((mcs > 0).sum()) > 20
