@@ -324,6 +324,16 @@ int seg_width(int E, int rb0, int occ, bool dl) {
     return rb;
 }
 
+// INET_NR_LANES in the environment: the lanes per env instead of seg_width's (envs of up to 64 robots), a power of two
+// from next_pow2(R) to 64, so that a layout that the rule gives to large batches can be run and compared on small ones.
+// 0: not such a number.
+int lanes_from_env(int rb0, int rb) {
+    const char* v = getenv("INET_NR_LANES");
+    if (!v || rb0 > inet::STEP_WAVE) return rb;
+    const int n = atoi(v);
+    return n >= rb0 && n <= inet::STEP_WAVE && (n & (n - 1)) == 0 ? n : 0;
+}
+
 // the argument checks and the launch of one step kernel (UL: dl NULL)
 int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const InetNrTables* tab,
                            const InetNrParams* prm, const InetNrRow* rows, int32_t n_rows, int64_t T, const float* x,
@@ -352,7 +362,9 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
         return INET_NR_EINVAL;
     const int n_data = p.n_data > 0 ? p.n_data : n_rows;
     const bool ir = p.comb == 2, vref = p.input_kind == 2;
-    const int rb = seg_width(p.E, next_pow2(p.R), cells ? 1 : 2, dl != nullptr);
+    const int rb0 = next_pow2(p.R);
+    const int rb = lanes_from_env(rb0, seg_width(p.E, rb0, cells ? 1 : 2, dl != nullptr));
+    if (rb == 0) return INET_NR_EINVAL;
     // the single-cell entry points run one cell; inet_nr_step_cells several
     if ((cells != nullptr) != (p.n_cells > 1)) return INET_NR_EINVAL;
     inet::StepFn fn;
