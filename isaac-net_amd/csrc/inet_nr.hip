@@ -303,27 +303,6 @@ bool rlf_ok(const InetNrCells& c, bool step) {
 
 int next_pow2(int v) { int p = 1; while (p < v) p <<= 1; return p; }
 
-// The lanes of a wavefront that one env of next_pow2(R) = rb0 lanes takes: rb0, or twice, four times, ... that while the
-// batch still leaves the chip room. A wavefront's time is its serial chain of slots, and the work that its envs deal
-// over the 64 lanes (fading draws, estimates, the MCS search) grows with the envs it holds, so a batch that does not
-// fill the chip is spread over more wavefronts with fewer envs each, down to one env per wavefront. The room is one
-// wavefront for each of the 1024 SIMDs, or the `occ` that are resident on one; past one per SIMD an env takes at most
-// four times its own lanes, and the DL launch, whose short slots gain nothing, keeps to one per SIMD. Measured, us per
-// step in 8 / 16 / 32 / 64 lanes per env: 64 x 8 round robin 99.9 / 88.8 / 80.4 / 81.2, 2048 x 8 104 / 96 / 89 / 103;
-// default configuration 256 x 16 (20 UL slots) - / 1202 / 679 / 495, 2048 x 16 (8 UL slots) - / 579 / 328 / 276,
-// 4096 x 16 - / 573 / 371 / 511, 1024 x 32 - / - / 364 / 264, 4096 x 32 - / - / 443 / 575; UL and DL 2048 x 32
-// - / - / 524 / 544; three cells (one wavefront per SIMD) 1024 x 16 - / 728 / 552 / 354, 2048 x 32 - / - / 813 / 894.
-int seg_width(int E, int rb0, int occ, bool dl) {
-    constexpr int64_t SIMDS = 1024;
-    int rb = rb0;
-    while (rb < inet::STEP_WAVE) {
-        const int64_t waves = ((int64_t)E * 2 * rb + inet::STEP_WAVE - 1) / inet::STEP_WAVE;
-        if (waves > SIMDS && (dl || 2 * rb > 4 * rb0 || waves > occ * SIMDS)) break;
-        rb *= 2;
-    }
-    return rb;
-}
-
 // INET_NR_LANES in the environment: the lanes per env instead of seg_width's (envs of up to 64 robots), a power of two
 // from next_pow2(R) to 64, so that a layout that the rule gives to large batches can be run and compared on small ones.
 // 0: not such a number.
@@ -362,16 +341,22 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
         return INET_NR_EINVAL;
     const int n_data = p.n_data > 0 ? p.n_data : n_rows;
     const bool ir = p.comb == 2, vref = p.input_kind == 2;
-    const int rb0 = next_pow2(p.R);
-    const int rb = lanes_from_env(rb0, seg_width(p.E, rb0, cells ? 1 : 2, dl != nullptr));
-    if (rb == 0) return INET_NR_EINVAL;
     // the single-cell entry points run one cell; inet_nr_step_cells several
     if ((cells != nullptr) != (p.n_cells > 1)) return INET_NR_EINVAL;
-    inet::StepFn fn;
     // the builds with the common switches fixed at compile time (INET_NR_GENERIC=1 keeps the general build, for
     // comparing the two)
     const char* gen = getenv("INET_NR_GENERIC");
     const int fx = (gen && gen[0] == '1') ? 0 : inet::fx_profile(p);
+    // the DL link resolves frame completion in the slot loop: no per-slot history in LDS
+    const int n_hist = dl ? 0 : n_data, nc = cells ? cells->C : 1;
+    const int rb0 = next_pow2(p.R);
+    const int rb = lanes_from_env(rb0, inet::seg_width(p.E, rb0, cells ? 1 : 2, dl != nullptr, [&](int w) {
+        const bool common = !cells && inet::step_common(p.P, ir, vref, w, fx);
+        return inet::step_lds_static(p.S, nc, ir, common) +
+               inet::step_lds_bytes(common ? 0 : n_hist, p.harq_drop, w, p.max_tx, nc, p.S);
+    }));
+    if (rb == 0) return INET_NR_EINVAL;
+    inet::StepFn fn;
     if (cells) {
         const InetNrCells& c = *cells;
         if (c.C != p.n_cells || c.C > INET_NR_MAX_C || (p.input_kind != 0 && p.input_kind != 3) || p.F > 64 || dl)
@@ -392,11 +377,9 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
     InetNrArrivals none{};
     if (arr && (!arr->counts || !arr->sizes || arr->n_cls <= 0 || (arr->pkt_overhead && arr->pkt_payload <= 0)))
         return INET_NR_EINVAL;
-    // the DL link resolves frame completion in the slot loop: no per-slot history in LDS
-    const int n_hist = dl ? 0 : n_data;
     inet::StepArgs a{*st, dl, cells, t, p, rows, n_rows, n_hist, arr ? *arr : none, T, x, cur_hid, *out, rb,
                      (unsigned)((p.E + envs_pw - 1) / envs_pw),
-                     inet::step_lds_bytes(n_hist, p.harq_drop, rb, p.max_tx, cells ? cells->C : 1, p.S),
+                     inet::step_lds_bytes(n_hist, p.harq_drop, rb, p.max_tx, nc, p.S),
                      inet::step_lds_bytes(0, p.harq_drop, rb, p.max_tx),
                      (hipStream_t)stream};
     // several cells: the static LDS grows with the cells (each lane's fading normals, 2 NC S floats, the

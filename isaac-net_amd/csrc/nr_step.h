@@ -28,6 +28,7 @@
 #include "aten_sort.h"
 #include "doppler.h"
 #include "inet_nr_dev.h"
+#include "step_width.h"
 
 namespace inet {
 
@@ -75,10 +76,6 @@ static __device__ uint64_t g_phase_clk[INET_PH_WAVES * INET_NPH];
 #define INET_PHASE_READER(NAME)
 #endif
 
-constexpr int STEP_WAVE = 64;          // one wavefront per workgroup
-constexpr int MAX_UL_ROWS = 64;        // UL data slots per control step
-constexpr int MAX_M = 32;              // MCS table rows
-constexpr int MAX_EQW = INET_NR_MAX_P + 1;
 constexpr uint32_t CH_STEP = 2;
 
 // Loads and stores at a uniform base plus a 32-bit per-lane byte offset (global_load ... v_off, s[base]): every
@@ -273,16 +270,6 @@ DEV void segment_f(int tbs, float r32, float& cbs, float& ncb) {
     const int c = b <= kcb ? 1 : (bg2 ? (b + 3815) / 3816 : (b + 8423) / 8424);
     cbs = c > 1 ? (float)((double)(b + 24 * c) / (double)c) : (float)b;
     ncb = (float)c;
-}
-
-// Dynamic LDS of the step kernel, in ints: the in-order pointer after every UL slot [n_ul][64], with RLC drop the
-// byte range of a TB that exhausted its HARQ [n_ul][64] x 2, then the per-env HARQ histograms [64 / RB][3][max_tx + 1];
-// with several cells (nc > 1) then per env each gNB's N+I estimate and this slot's interference [64 / RB][2][nc S].
-inline size_t step_lds_bytes(int n_ul, int harq_drop, int rb, int max_tx, int nc = 1, int S = 0) {
-    const size_t cw = rb > STEP_WAVE ? (size_t)rb : (size_t)STEP_WAVE;     // lanes per workgroup
-    return sizeof(int) * ((size_t)n_ul * cw * (harq_drop ? 3 : 1) +
-                          (cw / rb) * 3 * (max_tx + 1) +
-                          (nc > 1 ? (cw / rb) * 2 * nc * S : 0));
 }
 
 // v[idx] of a register array indexed by a runtime value (a chain of selects, no scratch memory: the empty asm keeps
@@ -2574,6 +2561,10 @@ void launch_step_mc(const StepArgs& a) {
                        a.stream, kern_args<InetNrState>(a));
 }
 
+// whether a one-wavefront env runs in a common configuration's build
+inline bool step_common(int P, bool ir, bool vref, int rb, int fx) {
+    return fx != 0 && !ir && !vref && (P == 8 || P == 16) && (rb == 32 || rb == 64);
+}
 // every (P, IR, per-subband SNR) with a runtime segment width; plus, for segments of 32 lanes without IR or per-subband
 // input, a build with the width fixed at compile time, and the common configuration's builds
 template <int S>
@@ -2583,7 +2574,7 @@ StepFn pick_step_s(int P, bool ir, bool vref, int rb, int fx) {
     // scratch at these process counts; against it at the same width (13 RBGs): 16 processes, 256 x 16 in 64 lanes,
     // 20 UL slots, 612 -> 495 us; 1024 x 32 in 64 lanes, 8 UL slots, 328 -> 264 us, in 32 lanes 412 -> 364 us;
     // 8 processes, 1024 x 32 in 64 lanes, 10 UL slots, 198 -> 154 us.
-    if (fx != 0 && !ir && !vref) {
+    if (step_common(P, ir, vref, rb, fx)) {
         if (P == 8 && rb == 32) return &launch_step<S, 8, false, false, 32, 1>;
         if (P == 8 && rb == 64) return &launch_step<S, 8, false, false, 64, 1>;
         if (P == 16 && rb == 32) return &launch_step<S, 16, false, false, 32, 1>;
