@@ -2565,8 +2565,11 @@ void launch_step_mc(const StepArgs& a) {
 inline bool step_common(int P, bool ir, bool vref, int rb, int fx) {
     return fx != 0 && !ir && !vref && (P == 8 || P == 16) && (rb == 32 || rb == 64);
 }
-// every (P, IR, per-subband SNR) with a runtime segment width; plus, for segments of 32 lanes without IR or per-subband
-// input, a build with the width fixed at compile time, and the common configuration's builds
+// every (P, IR, per-subband SNR) with a runtime segment width; plus, for segments of 32 and 64 lanes without IR or
+// per-subband input, builds with the width fixed at compile time (64 lanes at a runtime width / a fixed one, 13 RBGs:
+// 4 processes 1024 x 32 202 / 181 us, 2048 x 32 218 / 196, round robin 1024 x 32 131 / 117, 16 processes with max C/I
+// 1024 x 32 260 / 230; without it 2048 x 32 at 4 processes was faster in 32 lanes, 207), and the common configuration's
+// builds
 template <int S>
 StepFn pick_step_s(int P, bool ir, bool vref, int rb, int fx) {
     // the common configuration (with or without the Rician phasor) at 8 or 16 HARQ processes in segments of 32 or 64
@@ -2583,6 +2586,7 @@ StepFn pick_step_s(int P, bool ir, bool vref, int rb, int fx) {
 #define INET_PICK(PP)                                                                                 \
     if (P == PP) {                                                                                    \
         if (!ir && !vref && rb == 32) return &launch_step<S, PP, false, false, 32>;                  \
+        if (!ir && !vref && rb == 64) return &launch_step<S, PP, false, false, 64>;                  \
         return ir ? (vref ? &launch_step<S, PP, true, true, 0> : &launch_step<S, PP, true, false, 0>) \
                   : (vref ? &launch_step<S, PP, false, true, 0> : &launch_step<S, PP, false, false, 0>); \
     }
