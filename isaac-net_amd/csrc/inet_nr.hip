@@ -350,7 +350,7 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
     // the DL link resolves frame completion in the slot loop: no per-slot history in LDS
     const int n_hist = dl ? 0 : n_data, nc = cells ? cells->C : 1;
     const int rb0 = next_pow2(p.R);
-    const int rb = lanes_from_env(rb0, inet::seg_width(p.E, rb0, cells ? 1 : 2, dl != nullptr, [&](int w) {
+    const int rb = lanes_from_env(rb0, inet::seg_width(p.E, rb0, cells ? 1 : 2, [&](int w) {
         const bool common = !cells && inet::step_common(p.P, ir, vref, w, fx);
         return inet::step_lds_static(p.S, nc, ir, common) +
                inet::step_lds_bytes(common ? 0 : n_hist, p.harq_drop, w, p.max_tx, nc, p.S);

@@ -2573,10 +2573,11 @@ inline bool step_common(int P, bool ir, bool vref, int rb, int fx) {
 template <int S>
 StepFn pick_step_s(int P, bool ir, bool vref, int rb, int fx) {
     // the common configuration (with or without the Rician phasor) at 8 or 16 HARQ processes in segments of 32 or 64
-    // lanes. The general build keeps every switch's branch and scalar registers live and spills 264..456 B per lane to
+    // lanes. The general build keeps every switch's branch and scalar registers live and spills 96..424 B per lane to
     // scratch at these process counts; against it at the same width (13 RBGs): 16 processes, 256 x 16 in 64 lanes,
-    // 20 UL slots, 612 -> 495 us; 1024 x 32 in 64 lanes, 8 UL slots, 328 -> 264 us, in 32 lanes 412 -> 364 us;
-    // 8 processes, 1024 x 32 in 64 lanes, 10 UL slots, 198 -> 154 us.
+    // 20 UL slots, 432 -> 348 us; 1024 x 32 in 64 lanes, 8 UL slots, 239 -> 198 us, in 32 lanes 316 -> 261 us;
+    // 8 processes, 1024 x 32 in 64 lanes, 10 UL slots, 185 -> 157 us, 4096 x 32 in 32 lanes 240 -> 207 us; UL and DL
+    // 4096 x 32 584 -> 498 us; 18 RBGs at 16 processes, 4096 x 32, 375 -> 237 us.
     if (step_common(P, ir, vref, rb, fx)) {
         if (P == 8 && rb == 32) return &launch_step<S, 8, false, false, 32, 1>;
         if (P == 8 && rb == 64) return &launch_step<S, 8, false, false, 64, 1>;
@@ -2632,8 +2633,8 @@ template <int S>
 StepFn pick_step_w2_s(int P, bool ir, int fx) {
     if constexpr (S == 8)                            // config 5's switches without the Rician phasor, 8 HARQ
         if (fx == 2 && P == 8 && !ir) return &launch_step_w2<8, 8, false, 2>;
-    // the common configuration (13 RBGs, 16 processes, 4096 x 100, 8 UL slots: 1863 us in the general build, with 392 B
-    // per lane of scratch, 1593 us in this one)
+    // the common configuration (13 RBGs, 4096 x 100: 16 processes, 8 UL slots, 1590 us in the general build, 1358 us in
+    // this one; 8 processes, 10 UL slots, 1474 and 1238 us)
     if (fx != 0 && P == 8 && !ir) return &launch_step_w2<S, 8, false, 1>;
     if (fx != 0 && P == 16 && !ir) return &launch_step_w2<S, 16, false, 1>;
 #define INET_PICK_W2(PP) \

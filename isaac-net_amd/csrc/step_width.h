@@ -38,24 +38,24 @@ inline size_t step_lds_static(int S, int nc, bool ir, bool common) {
 // fill the chip is spread over more wavefronts with fewer envs each, down to one env per wavefront. The room is the
 // wavefronts that are resident at once: one for each of the 1024 SIMDs, or the `occ` that its registers hold, and no more
 // than the 160 KiB of a CU hold at lds(rb) bytes each (in allocations of 1280): one wavefront beyond it is a second
-// round of the whole chain. Past one per SIMD an env takes at most four times its own lanes, and the DL launch keeps to
-// one per SIMD. Measured, us per step in 8 / 16 / 32 / 64 lanes per env, beside the wavefronts resident at 64:
-// 64 x 8 round robin 99.9 / 88.8 / 80.4 / 81.2, 2048 x 8 104 / 96 / 89 / 103 (2048); default configuration 256 x 16
-// (20 UL slots) - / 1202 / 679 / 495, 2048 x 16 (8 UL slots) - / 579 / 328 / 276, 4096 x 16 - / 573 / 371 / 511,
-// 1024 x 32 - / - / 364 / 264, 4096 x 32 - / - / 443 / 575 (2048); UL and DL 2048 x 32 - / - / 524 / 544; three cells
-// 1024 x 16 - / 728 / 552 / 354, 2048 x 32 - / - / 813 / 894 (1024). Where LDS holds fewer: RLC UM (the losses of every
-// slot in LDS), 20 UL slots, 16 processes, 2048 x 32 - / - / 713 / 1220, 4096 x 8 801 / 630 / 1044 / 1715 (1280); seven
-// cells 1024 x 32 - / - / 1382 / 1830, 2048 x 8 1317 / 973 / 1493 / 2174 (512); four cells 1024 x 16 - / 843 / 635 / 831
-// (768).
+// round of the whole chain. Measured, us per step in 8 / 16 / 32 / 64 lanes per env, and the wavefronts resident:
+//   two per SIMD, 2048: round robin 512 x 8 105 / 95 / 84 / 82, 2048 x 8 107 / 99 / 90 / 91, 4096 x 8 115 / 105 / 99 /
+//   164; default configuration (8 UL slots) 256 x 16 - / 313 / 196 / 159, 2048 x 16 - / 344 / 209 / 195, 4096 x 16
+//   - / 349 / 248 / 370, 1024 x 32 - / - / 257 / 193, 4096 x 32 - / - / 321 / 437; UL and DL 4096 x 8 421 / 400 / 322 /
+//   535, 2048 x 32 - / - / 446 / 437, 4096 x 32 - / - / 494 / 801
+//   one per SIMD, 1024: three cells 1024 x 16 - / 690 / 527 / 335, 2048 x 32 - / - / 736 / 836
+//   fewer by LDS: RLC UM (the losses of every slot in LDS) over 20 UL slots at 16 processes, 1280: 2048 x 32 - / - / 713 /
+//   1103, 4096 x 8 797 / 629 / 1044 / 1556; four cells, 768: 1024 x 16 - / 840 / 634 / 833; seven cells, 512: 1024 x 32
+//   - / - / 1382 / 1830, 2048 x 8 1314 / 974 / 1495 / 2171
 template <class L>
-int seg_width(int E, int rb0, int occ, bool dl, L lds) {
-    constexpr int64_t CUS = 256, SIMDS = 4 * CUS, LDS = 160 * 1024;
+int seg_width(int E, int rb0, int occ, L lds) {
+    constexpr int64_t CUS = 256, LDS = 160 * 1024;
     int rb = rb0;
     while (rb < STEP_WAVE) {
         const int64_t waves = ((int64_t)E * 2 * rb + STEP_WAVE - 1) / STEP_WAVE;
         const int64_t need = ((int64_t)lds(2 * rb) + 1279) / 1280 * 1280, held = need > 0 ? LDS / need : 0;
         const int64_t room = CUS * (held < 4 * occ ? held : 4 * occ);
-        if (waves > room || (waves > SIMDS && (dl || 2 * rb > 4 * rb0))) break;
+        if (waves > room) break;
         rb *= 2;
     }
     return rb;
