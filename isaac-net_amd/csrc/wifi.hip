@@ -330,7 +330,10 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
     float* s_fin = s_rem + F8 * WAVE;                     // [F][64] finish time, then the compaction staging row
     uint8_t* s_cls = (uint8_t*)(s_fin + F * WAVE);        // [F][64] class of every frame slot
     uint8_t* s_src = s_cls + F * WAVE;                    // [F][64] source slot of every compacted slot
-    int32_t* s_stage = (int32_t*)s_fin;
+    // (the staging row holds words of any field, a word of the lane's own column each, as the bits of a float: one
+    // element type for all of its accesses)
+    auto stage = [&](int f, int32_t v) { s_fin[f * WAVE + (int)threadIdx.x] = __int_as_float(v); };
+    auto staged = [&](int f) -> int32_t { return __float_as_int(s_fin[f * WAVE + (int)threadIdx.x]); };
 
     // the enqueue's global calls are counted by a workgroup of their own, the first (a one-wave pass over every count,
     // beside the others' steps: behind a step it lengthened the whole launch)
@@ -1000,7 +1003,7 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
                 if (gone) s_rem[o] = 0.0f;
                 if (!gone && cap >= 0) vmask |= 1ull << f;
                 if (dt && !gone) dmask |= 1ull << f;
-                s_stage[o] = gone ? -1 : cap;              // the new cap row, staged for the permutation
+                stage(f, gone ? -1 : cap);                 // the new cap row, staged for the permutation
             }
         if (!rob) continue;
         if (vec) {
@@ -1041,7 +1044,7 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
     if (__ballot(moves) == 0ull) {
         if (rob)
             for (int f = 0; f < F; ++f) {
-                st.cap[fo + (size_t)f * R] = s_stage[f * WAVE + lane];
+                st.cap[fo + (size_t)f * R] = staged(f);
                 st.det[fo + (size_t)f * R] = (uint8_t)((dmask >> f) & 1ull);
                 st.rem[fo + (size_t)f * R] = s_rem[f * WAVE + lane];
             }
@@ -1054,22 +1057,27 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
         // cap (staged above), then every other field through the staging row
         for (int gdst = 0; gdst < F; ++gdst) {
             const int sf = s_src[gdst * WAVE + lane];
-            st.cap[fo + (size_t)gdst * R] = s_stage[sf * WAVE + lane];
+            st.cap[fo + (size_t)gdst * R] = staged(sf);
             st.det[fo + (size_t)gdst * R] = (uint8_t)((dmask >> sf) & 1ull);
         }
         auto permute = [&](auto* p) {
             using T = std::remove_reference_t<decltype(*p)>;
-            T* const s_t = reinterpret_cast<T*>(s_stage);
             for (int f0 = 0; f0 < F; f0 += 8) {
                 T v[8];
 #pragma unroll
                 for (int l = 0; l < 8; ++l) v[l] = p[fo + (size_t)(f0 + l < F ? f0 + l : F - 1) * R];
 #pragma unroll
                 for (int l = 0; l < 8; ++l)
-                    if (f0 + l < F) s_t[(f0 + l) * WAVE + lane] = v[l];
+                    if (f0 + l < F) {
+                        if constexpr (std::is_same<T, float>::value) stage(f0 + l, __float_as_int(v[l]));
+                        else stage(f0 + l, (int32_t)v[l]);
+                    }
             }
-            for (int gdst = 0; gdst < F; ++gdst)
-                p[fo + (size_t)gdst * R] = s_t[s_src[gdst * WAVE + lane] * WAVE + lane];
+            for (int gdst = 0; gdst < F; ++gdst) {
+                const int32_t w = staged(s_src[gdst * WAVE + lane]);
+                if constexpr (std::is_same<T, float>::value) p[fo + (size_t)gdst * R] = __int_as_float(w);
+                else p[fo + (size_t)gdst * R] = (T)w;
+            }
         };
         if (moves) {
             permute(st.cls);
@@ -1078,10 +1086,9 @@ __global__ __launch_bounds__(WAVE) void wifi_step_kernel(InetWifiState st, InetW
             permute(st.f_own);
             permute(st.f_snr);
         }
-        float* s_stf = (float*)s_stage;
-        for (int f = 0; f < F; ++f) s_stf[f * WAVE + lane] = s_rem[f * WAVE + lane];
+        for (int f = 0; f < F; ++f) stage(f, __float_as_int(s_rem[f * WAVE + lane]));
         for (int gdst = 0; gdst < F; ++gdst) {
-            const float v = s_stf[s_src[gdst * WAVE + lane] * WAVE + lane];
+            const float v = __int_as_float(staged(s_src[gdst * WAVE + lane]));
             st.rem[fo + (size_t)gdst * R] = v;
             s_rem[gdst * WAVE + lane] = v;
         }
