@@ -279,7 +279,7 @@ def run_wifi(args, P, torch):
                                   "7 attempts), 802.11ax 20 MHz 12 MCS, "
                                   + ("per-slot CSMA/CA over the 20 ms step" if slots else f"K={K} sub-steps of 1 ms")
                                   + ", 1500 B @0.4 per station-step, FIFO 16, 50 m disc, log-distance + shadowing",
-                      "envs": E, "stations": R, "substeps_per_step": K, "envs_per_wave": args.envs_per_wave,
+                      "envs": E, "stations": R, "substeps_per_step": K, "envs_per_wave": eng.envs_per_wave,
                       "parallelism": "single GPU",
                       "launch": "eager, one launch per step (the enqueue in the step kernel), static output "
                                 "buffers overwritten by every step (as the reference's graph backend returns them)"},
@@ -287,7 +287,7 @@ def run_wifi(args, P, torch):
            "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_GBS, "unit": "GB/s",
                         "frac": achieved / PEAK_GBS, "kernel": "wifi_step_kernel",
                         "kernel_ms_avg": k_avg, "kernel_ms_median": k_ms[len(k_ms) // 2],
-                        **measured_fields(f"wifi_step_kernel_counters_{args.workload}_epw{args.envs_per_wave}"
+                        **measured_fields(f"wifi_step_kernel_counters_{args.workload}_epw{eng.envs_per_wave}"
                                           if (E, R) == (2048, 16) else "", k_avg),
                         "kernel_timing": "HIP events around each launch on the launch stream, the timed loop's "
                                          "launches repeated behind a GPU spin",
@@ -651,7 +651,8 @@ def main():
                          "inputs")
     ap.add_argument("--envs", type=int, default=None)
     ap.add_argument("--robots", type=int, default=None)
-    ap.add_argument("--envs-per-wave", type=int, default=1, help="level WIFI: envs per 64-lane wavefront")
+    ap.add_argument("--envs-per-wave", type=int, default=None,
+                    help="Wi-Fi levels: envs per 64-lane wavefront (default: the engine's own choice)")
     ap.add_argument("--out-format", default="reference", choices=("reference", "compact"))
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--graph", action="store_true",

@@ -286,8 +286,8 @@ DEV T sel_of(const T (&v)[N], int idx) {
     return r;
 }
 
-// The step kernel's arguments, one struct at the start of the kernel argument segment. lk is the DL link's state (the UL
-// build reads st; its lk holds nothing).
+// The step kernel's arguments, one struct at the start of the kernel argument segment. lk is the DL link's state (the
+// UL build reads st; its lk holds nothing).
 struct NoLink {};
 template <class LS>
 struct StepKernArgs {
@@ -306,9 +306,9 @@ struct StepKernArgs {
 };
 // The kernel's arguments read again from here on: the empty asm hides that the address is the one the kernel began
 // with, so the fields come from the scalar cache where they are used instead of being held in scalar registers since
-// the kernel's start: they do not fit, and a spilled one costs a lane read and a hazard wait at each use. Read again for the end of
-// the step and in every slot, the common build at 13 RBGs spills 86 scalars instead of 233: rl 4096 x 32 216.4 -> 211.2
-// us, 3000 x 20 at 14 RBGs 171.0 -> 161.5, 16384 x 128 2625 -> 2574.
+// the kernel's start: they do not fit, and a spilled one costs a lane read and a hazard wait at each use. Read again for
+// the end of the step and in every slot: the common build at 13 RBGs spilled 233 scalars before and 86 after, rl 4096 x
+// 32 216.4 -> 211.2 us, 3000 x 20 at 14 RBGs 171.0 -> 161.5, 16384 x 128 2625 -> 2574 (the present one spills 115).
 template <class LS>
 DEV const StepKernArgs<LS>& args_again() {
     const __attribute__((address_space(4))) char* p =
@@ -317,8 +317,8 @@ DEV const StepKernArgs<LS>& args_again() {
     return *(const StepKernArgs<LS>*)p;
 }
 
-// The builds that complete frames as the in-order pointer passes them: the common configuration in one cell (no losses to
-// place among the slots). The history's 4 B per lane and slot bound the workgroups of a CU, and its replay costs
+// The builds that complete frames as the in-order pointer passes them: the common configuration in one cell (no losses
+// to place among the slots). The history's 4 B per lane and slot bound the workgroups of a CU, and its replay costs
 // frames x slots: 16384 x 128 (20 UL slots) 1712 -> 1558 us, the default configuration 1024 x 32 (20 UL slots, long
 // queues) 434 -> 413, 4096 x 100 1371 -> 1355, rl 4096 x 32 205.8 -> 204.4 (same card).
 constexpr bool step_walks(int NC, int FX) { return NC == 1 && FX != 0; }
@@ -338,8 +338,8 @@ constexpr bool step_walks(int NC, int FX) { return NC == 1 && FX != 0; }
 //
 // FX = 1 builds the kernel for the common configuration (PF, chase combining, EESM, RLC AM, OLLA, PHR cap, retx
 // priority, fading, with a fixed Rician phasor or without: then its K and phasor are 0, and the gain's 0 0 + 1 h is h
-// bit for bit; fx_profile), FX = 2 for the same without the Rician phasor: those switches become compile-time constants, which removes their tests from the slot loop and the scalar registers that
-// hold them.
+// bit for bit; fx_profile), FX = 2 for the same without the Rician phasor: those switches become compile-time
+// constants, which removes their tests from the slot loop and the scalar registers that hold them.
 // Minimum waves per SIMD (the register budget): 2, and 3 for the two-wave FX = 2 build (envs of 65..128 robots at the
 // common configuration, 8 RBGs and processes: 168 VGPRs with 72 B per lane of spills, 1558 us on 16384 x 128 against
 // 1867 for 204 VGPRs at 2 waves; 4 waves, at 128 VGPRs and 232 B, take 2427. 13 RBGs with 16 processes at 3 waves spill
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     // per HARQ process: its state word, first byte and ready slot. The words that only a transmission of the process
     // touches (its last byte, TBS, combined SINR, IR sums) stay in memory: a retransmission reads them, a transmission
     // writes them. In registers they took 3 P (IR: 5 P) of the 256, spilled at 16 processes and with two waves per env
-    // (120 and 108 B per lane of scratch, now 0 and 52), and were read and written whole: 4096 x 100 at 16 processes
+    // (120 and 108 B per lane of scratch, 0 and 52 without them), and were read and written whole: 4096 x 100 at 16 processes
     // 1563 -> 1371 us, 16384 x 128 1964 -> 1712, rl 4096 x 32 210.5 -> 203.6, HARQ-IR 1024 x 16 243 -> 226.
     uint32_t hmeta[P];
     int hlo[P], hrdy[P];
@@ -2524,7 +2524,8 @@ template <int S, int P, bool IR, bool VREF, int RBT, int FX = 0>
 void launch_step(const StepArgs& a) {
     if (a.dl)
         hipLaunchKernelGGL((nr_step_kernel<S, P, IR, VREF, RBT, InetNrDlState, 1, FX>), dim3(a.grid),
-                           dim3(STEP_WAVE), (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrDlState>(a));
+                           dim3(STEP_WAVE), (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream,
+                           kern_args<InetNrDlState>(a));
     else
         hipLaunchKernelGGL((nr_step_kernel<S, P, IR, VREF, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(STEP_WAVE),
                            (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrState>(a));
@@ -2550,15 +2551,15 @@ void launch_step_w2(const StepArgs& a) {
                                (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrDlState>(a));
             return;
         }
-    hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(RBT), (step_walks(1, FX) ? a.lds_walk : a.lds),
-                       a.stream, kern_args<InetNrState>(a));
+    hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, 1, FX>), dim3(a.grid), dim3(RBT),
+                       (step_walks(1, FX) ? a.lds_walk : a.lds), a.stream, kern_args<InetNrState>(a));
 }
 
 // the multi-cell step: NC cells, pose input, runtime segment width (RBT = 0) or one fixed at compile time
 template <int S, int P, bool IR, int NC, int FX = 0, int RBT = 0>
 void launch_step_mc(const StepArgs& a) {
-    hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, NC, FX>), dim3(a.grid), dim3(STEP_WAVE), a.lds,
-                       a.stream, kern_args<InetNrState>(a));
+    hipLaunchKernelGGL((nr_step_kernel<S, P, IR, false, RBT, InetNrState, NC, FX>), dim3(a.grid), dim3(STEP_WAVE),
+                       a.lds, a.stream, kern_args<InetNrState>(a));
 }
 
 // whether a one-wavefront env runs in a common configuration's build

@@ -5,9 +5,9 @@
 // Every element is read unconditionally, in blocks of 8, from a row that is padded with zeros to whole blocks, and the
 // blocks that a length has are chosen by branches on the length alone. (One masked add per element, the form that
 // this replaces, kept a lane mask per element and per call site alive over the whole step: 1066 spilled scalar
-// registers in the Wi-Fi mean-field step, read back by lane reads in every sub-step, and more than 256 vector registers,
-// one wavefront per SIMD; now 209, and two. 2048 envs of 16 robots, one env per wavefront: 437 us a step before, 278
-// after.) A zero added to a partial sum changes no bit of it: the sums begin at +0.0, so none is -0.0.
+// registers in the Wi-Fi mean-field step at one AP, read back by lane reads in every sub-step, and 276 vector
+// registers, one wavefront per SIMD; the present step spills 164 and has 175, two wavefronts. 2048 envs of 16 robots,
+// one env per wavefront: 437 us a step before, 278 after.) A zero added to a partial sum changes no bit of it: the sums begin at +0.0, so none is -0.0.
 #pragma once
 
 #ifdef __HIPCC__

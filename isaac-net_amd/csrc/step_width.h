@@ -32,21 +32,22 @@ inline size_t step_lds_static(int S, int nc, bool ir, bool common) {
                           (ir ? MAX_M * MAX_EQW : 1) + MAX_UL_ROWS + 24 + (nc > 1 ? q * (1 + 2 * nc) + nc * cw : 2));
 }
 
-// The lanes of a wavefront that one env of next_pow2(R) = rb0 lanes takes: rb0, or twice, four times, ... that while the
-// batch still leaves the chip room. A wavefront's time is its serial chain of slots, and the work that its envs deal
-// over the 64 lanes (fading draws, estimates, the MCS search) grows with the envs it holds, so a batch that does not
-// fill the chip is spread over more wavefronts with fewer envs each, down to one env per wavefront. The room is the
-// wavefronts that are resident at once: one for each of the 1024 SIMDs, or the `occ` that its registers hold, and no more
-// than the 160 KiB of a CU hold at lds(rb) bytes each (in allocations of 1280): one wavefront beyond it is a second
-// round of the whole chain. Measured, us per step in 8 / 16 / 32 / 64 lanes per env, and the wavefronts resident:
-//   two per SIMD, 2048: round robin 512 x 8 105 / 95 / 84 / 82, 2048 x 8 107 / 99 / 90 / 91, 4096 x 8 115 / 105 / 99 /
-//   164; default configuration (8 UL slots) 256 x 16 - / 313 / 196 / 159, 2048 x 16 - / 344 / 209 / 195, 4096 x 16
-//   - / 349 / 248 / 370, 1024 x 32 - / - / 257 / 193, 4096 x 32 - / - / 321 / 437; UL and DL 4096 x 8 421 / 400 / 322 /
-//   535, 2048 x 32 - / - / 446 / 437, 4096 x 32 - / - / 494 / 801
-//   one per SIMD, 1024: three cells 1024 x 16 - / 690 / 527 / 335, 2048 x 32 - / - / 736 / 836
-//   fewer by LDS: RLC UM (the losses of every slot in LDS) over 20 UL slots at 16 processes, 1280: 2048 x 32 - / - / 713 /
-//   1103, 4096 x 8 797 / 629 / 1044 / 1556; four cells, 768: 1024 x 16 - / 840 / 634 / 833; seven cells, 512: 1024 x 32
-//   - / - / 1382 / 1830, 2048 x 8 1314 / 974 / 1495 / 2171
+// The lanes of a wavefront that one env of next_pow2(R) = rb0 lanes takes: rb0, or twice, four times, ... that while
+// the batch still leaves the chip room. A wavefront's time is its serial chain of slots, and the work that its envs
+// deal over the 64 lanes (fading draws, estimates, the MCS search) grows with the envs it holds, so a batch that does
+// not fill the chip is spread over more wavefronts with fewer envs each, down to one env per wavefront. The room is
+// the wavefronts that are resident at once: one for each of the 1024 SIMDs, or the `occ` that its registers hold, and
+// no more than the 160 KiB of a CU hold at lds(rb) bytes each (in allocations of 1280): one wavefront beyond it is a
+// second round of the whole chain. Measured, us per step in 8 / 16 / 32 / 64 lanes per env, by the wavefronts
+// resident at 64:
+//   2048, two per SIMD: round robin 512 x 8 105 / 95 / 84 / 82, 2048 x 8 107 / 99 / 90 / 91, 4096 x 8 115 / 105 / 99
+//   / 164; default configuration (8 UL slots) 256 x 16 - / 313 / 196 / 159, 2048 x 16 - / 344 / 209 / 195, 4096 x 16
+//   - / 349 / 248 / 370, 1024 x 32 - / - / 257 / 193, 4096 x 32 - / - / 321 / 437; UL and DL 4096 x 8 421 / 400 / 322
+//   / 535, 2048 x 32 - / - / 446 / 437, 4096 x 32 - / - / 494 / 801
+//   1024, one per SIMD: three cells 1024 x 16 - / 690 / 527 / 335, 2048 x 32 - / - / 736 / 836
+//   fewer by LDS: RLC UM (the losses of every slot in LDS) over 20 UL slots at 16 processes, 1280: 2048 x 32 - / - /
+//   713 / 1103, 4096 x 8 797 / 629 / 1044 / 1556; four cells, 768: 1024 x 16 - / 840 / 634 / 833; seven cells, 512:
+//   1024 x 32 - / - / 1382 / 1830, 2048 x 8 1314 / 974 / 1495 / 2171
 template <class L>
 int seg_width(int E, int rb0, int occ, L lds) {
     constexpr int64_t CUS = 256, LDS = 160 * 1024;

@@ -125,7 +125,7 @@ class HipWifiEngine:
 
     def _auto_envs_per_wave(self, rb):
         """The launch's envs per wavefront, in segments of rb = next_pow2(R) lanes (mean-field: of next_pow2(R + A)):
-        the fewest with which every wavefront of the batch is resident, or all that fit."""
+        the fewest that leave at most _waves wavefronts, or all that fit."""
         seg = rb if self.level == "WIFI_DCF" else min(64, 1 << (self.R + self.A - 1).bit_length())
         g = 1
         while 2 * g * seg <= 64 and -(-self.E // g) > self._waves:
