@@ -2020,7 +2020,9 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     if (cl.use_int) x = x - ((10.0f * log10f(cl.noise_mw + s_if[serv * S + s])) - ni_la[s]);
                 nan |= x != x;
                 xs[s] = x;
-                if (!pm.eesm) s_x[s * CW + lane] = x;                    // (the mean-dB row)
+                // (the mean-dB row. Not with HARQ-IR, which decodes on the log-sum: the row lies over the pair list that
+                // held_lse writes before its first barrier, with an even RBG count over another wavefront's)
+                if constexpr (!IR) if (!pm.eesm) s_x[s * CW + lane] = x;
             }
             // the EESM log-sum of the held RBGs (lse_eesm of the linear SINR per RBG)
             const float lse_tx = (IR || pm.eesm) ? held_lse(tx, xs, mcs, nan) : 0.0f;
