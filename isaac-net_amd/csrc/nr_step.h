@@ -1571,7 +1571,7 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
             // free between the estimate and the allocation), walks the sorted order and marks the candidates whose
             // running RBG count fits. (Wave-uniform: every env of the wavefront takes part when any env needs it.)
             bool exact = false;
-            if constexpr (W == 1) exact = rb > 16 && __ballot(tie) != 0ull;
+            if constexpr (W == 1) exact = R > 16 && __ballot(tie) != 0ull;
             else if (ranked) exact = env_any(tie);          // (W > 1: one env per workgroup, `ranked` is uniform)
             if (exact) {
                 const int XS = NC * 3 * rb + rb + NC * 64;   // ints per env: NC (keys, indices, counts), marks, stacks
