@@ -389,7 +389,15 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
         const size_t nc = (size_t)cells->C, ns = (size_t)p.S;
         const size_t stat = sizeof(float) * (2 * nc * ns * inet::STEP_WAVE + nc * ns * (1 + 2 * nc) +
                                              nc * inet::STEP_WAVE) + 16384;
-        if (a.lds + stat > 160 * 1024) return INET_NR_EUNSUPPORTED;
+        if (a.lds + stat > inet::CU_LDS) return INET_NR_EUNSUPPORTED;
+    } else {
+        // one cell: four wavefronts per env with RLC UM's per-slot losses in LDS (256 lanes x 12 B a slot) leave room
+        // for 29..40 UL slots by RBG count; a launch beyond the CU's LDS aborts the queue
+        const bool walk = rb <= inet::STEP_WAVE ? inet::step_common(p.P, ir, vref, rb, fx)
+                                                : rb == 2 * inet::STEP_WAVE && fx != 0 && !ir && (p.P == 8 || p.P == 16);
+        const int W = rb > inet::STEP_WAVE ? rb / inet::STEP_WAVE : 1;
+        if (inet::step_lds_static(p.S, 1, ir, walk, W) + (walk ? a.lds_walk : a.lds) > inet::CU_LDS)
+            return INET_NR_EUNSUPPORTED;
     }
     fn(a);
     return hipGetLastError() == hipSuccess ? INET_NR_OK : INET_NR_ELAUNCH;

@@ -24,12 +24,15 @@ inline size_t step_lds_bytes(int n_ul, int harq_drop, int rb, int max_tx, int nc
                           (nc > 1 ? (cw / rb) * 2 * nc * S : 0));
 }
 
-// Static LDS of a one-wavefront build for S RBGs and nc cells: the kernel's __shared__ arrays, with room for their
-// alignment (the compiled kernels hold up to 100 B less). common: a build of the common configuration.
-inline size_t step_lds_static(int S, int nc, bool ir, bool common) {
-    const size_t q = (size_t)nc * S, cw = STEP_WAVE;
-    return sizeof(int) * ((2 * q + S) * cw + 11 * cw + 6 * MAX_M + 4 * S + 1 + (common ? 1 : S * S) +
-                          (ir ? MAX_M * MAX_EQW : 1) + MAX_UL_ROWS + 24 + (nc > 1 ? q * (1 + 2 * nc) + nc * cw : 2));
+constexpr size_t CU_LDS = 160 * 1024;
+
+// Static LDS of a build for S RBGs, nc cells and W wavefronts per env: the kernel's __shared__ arrays, with room for
+// their alignment (the compiled kernels hold up to 128 B less). common: a build of the common configuration.
+inline size_t step_lds_static(int S, int nc, bool ir, bool common, int W = 1) {
+    const size_t q = (size_t)nc * S, cw = (size_t)STEP_WAVE * W;
+    return sizeof(int) * ((2 * q + S) * cw + (W > 1 ? 13 : 11) * cw + 6 * MAX_M + 4 * S + 1 + (common ? 1 : S * S) +
+                          (ir ? MAX_M * MAX_EQW : 1) + MAX_UL_ROWS + 20 + 4 * W +
+                          (nc > 1 ? q * (1 + 2 * nc) + nc * cw : 2));
 }
 
 // The lanes of a wavefront that one env of next_pow2(R) = rb0 lanes takes: rb0, or twice, four times, ... that while
@@ -50,7 +53,7 @@ inline size_t step_lds_static(int S, int nc, bool ir, bool common) {
 //   1024 x 32 - / - / 1382 / 1830, 2048 x 8 1314 / 974 / 1495 / 2171
 template <class L>
 int seg_width(int E, int rb0, int occ, L lds) {
-    constexpr int64_t CUS = 256, LDS = 160 * 1024;
+    constexpr int64_t CUS = 256, LDS = CU_LDS;
     int rb = rb0;
     while (rb < STEP_WAVE) {
         const int64_t waves = ((int64_t)E * 2 * rb + STEP_WAVE - 1) / STEP_WAVE;

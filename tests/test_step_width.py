@@ -1,12 +1,14 @@
 """The lanes per env that the step launch gives a batch (csrc/step_width.h, compiled for the host with g++): wider than
 next_pow2(R) only while every wavefront of the batch is resident, by its registers and by its LDS; and the LDS that
 this counts on, against what the compiled kernels hold."""
+import ctypes
 import os
 import re
 import struct
 import subprocess
 
 import pytest
+import torch
 
 from conftest import ROOT
 from isaac_net_amd import _lib
@@ -18,11 +20,11 @@ DRIVER = r"""
 #include <cstdio>
 #include "step_width.h"
 int main() {
-    int E, rb0, occ, n_ul, drop, max_tx, nc, S, ir, common;
-    while (scanf("%d %d %d %d %d %d %d %d %d %d", &E, &rb0, &occ, &n_ul, &drop, &max_tx, &nc, &S, &ir,
-                 &common) == 10) {
+    int E, rb0, occ, n_ul, drop, max_tx, nc, S, ir, common, W;
+    while (scanf("%d %d %d %d %d %d %d %d %d %d %d", &E, &rb0, &occ, &n_ul, &drop, &max_tx, &nc, &S, &ir, &common,
+                 &W) == 11) {
         auto lds = [&](int w) {
-            return inet::step_lds_static(S, nc, ir, common) + inet::step_lds_bytes(n_ul, drop, w, max_tx, nc, S);
+            return inet::step_lds_static(S, nc, ir, common, W) + inet::step_lds_bytes(n_ul, drop, w, max_tx, nc, S);
         };
         const int rb = inet::seg_width(E, rb0, occ, lds);
         printf("%d", rb);
@@ -41,8 +43,9 @@ def width(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-std=c++17", f"-I{CSRC}", "-o", str(d / "drv"), str(d / "drv.cpp")], check=True)
 
     def run(rows):
-        """[(lanes, {width: LDS bytes of a wavefront})] of rows (E, rb0, occ, n_ul, drop, max_tx, nc, S, ir, common)."""
-        out = subprocess.run([str(d / "drv")], input="\n".join(" ".join(str(int(v)) for v in r) for r in rows),
+        """[(lanes, {width: LDS bytes of a wavefront})] of rows (E, rb0, occ, n_ul, drop, max_tx, nc, S, ir, common[, waves])."""
+        text = "\n".join(" ".join(str(int(v)) for v in (tuple(r) + (1,))[:11]) for r in rows)
+        out = subprocess.run([str(d / "drv")], input=text,
                              capture_output=True, text=True, check=True).stdout.split("\n")
         vals = [[int(v) for v in line.split()] for line in out if line]
         return [(v[0], {1 << i: b for i, b in enumerate(v[1:])}) for v in vals]
@@ -121,10 +124,25 @@ def test_static_lds_covers_the_compiled_kernels(width):
         m = pat.search(name)
         if m:
             S, _, ir, _, rbt, nc, fx = (int(v) for v in m.groups())
-            if rbt <= 64:
-                found.setdefault((S, nc, ir, int(fx != 0)), set()).add(lds)
-    assert {k[1] for k in found} == {1, 2, 3, 4, 5, 6, 7} and {k[0] for k in found if k[1] == 1} >= {8, 13, 18}
-    rows = [(1, 64, 1, 0, 0, -1, nc, S, ir, common) for S, nc, ir, common in found]
+            found.setdefault((S, nc, ir, int(fx != 0), max(1, rbt // 64)), set()).add(lds)
+    assert {k[4] for k in found} == {1, 2, 4} and {k[1] for k in found} == {1, 2, 3, 4, 5, 6, 7} and {k[0] for k in found if k[1] == 1} >= {8, 13, 18}
+    rows = [(1, 64, 1, 0, 0, -1, nc, S, ir, common, W) for S, nc, ir, common, W in found]
     for (k, have), (_, lds) in zip(found.items(), width(rows)):
         want = lds[64] - (8 * k[1] * k[0] if k[1] > 1 else 0)      # (less the N+I rows, dynamic)
         assert max(have) <= want <= min(have) + 128, (k, have, want)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="a refusal of the host's checks, tested where nothing can launch")
+@pytest.mark.parametrize("R,S,n_data,drop,rc", [(200, 16, 60, 1, -2), (200, 16, 20, 1, -3), (200, 18, 64, 0, -3),
+                                                (150, 13, 40, 1, -2), (100, 18, 64, 1, -3), (20, 18, 64, 1, -3)])
+def test_launch_beyond_the_lds_is_refused(R, S, n_data, drop, rc):
+    """Four wavefronts per env with RLC UM keep 3 KB of LDS per UL slot: with many slots the workgroup needs more than
+    a CU has, and the call is refused (-2) before the launch; what fits goes on to the launch (-3: no GPU here)."""
+    lib = _lib.load()
+    st, tb, pm, out = _lib.InetNrState(), _lib.InetNrTables(), _lib.InetNrParams(), _lib.InetNrOutputs()
+    tb.M, tb.C, tb.G, tb.EQW, tb.mcs_max, tb.NPRB = 29, 4, 8, 5, 28, 52
+    pm.E, pm.R, pm.S, pm.P, pm.F, pm.N = 2, R, S, 8, 16, 100
+    pm.max_tx, pm.input_kind, pm.harq_drop, pm.n_data, pm.n_cells = 4, 1, drop, n_data, 1
+    got = lib.inet_nr_step(ctypes.byref(st), ctypes.byref(tb), ctypes.byref(pm), ctypes.c_void_p(16), n_data, 0,
+                           ctypes.c_void_p(16), None, ctypes.byref(out), None)
+    assert got == rc
