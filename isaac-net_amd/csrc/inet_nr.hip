@@ -394,7 +394,8 @@ int32_t launch_step_kernel(const InetNrState* st, const InetNrDlState* dl, const
         // one cell: four wavefronts per env with RLC UM's per-slot losses in LDS (256 lanes x 12 B a slot) leave room
         // for 29..40 UL slots by RBG count; a launch beyond the CU's LDS aborts the queue
         const bool walk = rb <= inet::STEP_WAVE ? inet::step_common(p.P, ir, vref, rb, fx)
-                                                : rb == 2 * inet::STEP_WAVE && fx != 0 && !ir && (p.P == 8 || p.P == 16);
+                                                : rb == 2 * inet::STEP_WAVE && fx != 0 && !ir &&
+                                                      (p.P == 8 || p.P == 16);
         const int W = rb > inet::STEP_WAVE ? rb / inet::STEP_WAVE : 1;
         if (inet::step_lds_static(p.S, 1, ir, walk, W) + (walk ? a.lds_walk : a.lds) > inet::CU_LDS)
             return INET_NR_EUNSUPPORTED;

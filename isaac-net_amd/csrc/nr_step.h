@@ -306,8 +306,8 @@ struct StepKernArgs {
 };
 // The kernel's arguments read again from here on: the empty asm hides that the address is the one the kernel began
 // with, so the fields come from the scalar cache where they are used instead of being held in scalar registers since
-// the kernel's start: they do not fit, and a spilled one costs a lane read and a hazard wait at each use. Read again for
-// the end of the step and in every slot: the common build at 13 RBGs spilled 233 scalars before and 86 after, rl 4096 x
+// the kernel's start: they do not fit, and a spilled one costs a lane read and a hazard wait at each use. Read again
+// for the end of the step and in every slot: the common build at 13 RBGs spilled 233 scalars before and 86 after, rl 4096 x
 // 32 216.4 -> 211.2 us, 3000 x 20 at 14 RBGs 171.0 -> 161.5, 16384 x 128 2625 -> 2574 (the present one spills 115).
 template <class LS>
 DEV const StepKernArgs<LS>& args_again() {
@@ -485,8 +485,8 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
     // per HARQ process: its state word, first byte and ready slot. The words that only a transmission of the process
     // touches (its last byte, TBS, combined SINR, IR sums) stay in memory: a retransmission reads them, a transmission
     // writes them. In registers they took 3 P (IR: 5 P) of the 256, spilled at 16 processes and with two waves per env
-    // (120 and 108 B per lane of scratch, 0 and 52 without them), and were read and written whole: 4096 x 100 at 16 processes
-    // 1563 -> 1371 us, 16384 x 128 1964 -> 1712, rl 4096 x 32 210.5 -> 203.6, HARQ-IR 1024 x 16 243 -> 226.
+    // (120 and 108 B per lane of scratch, 0 and 52 without them), and were read and written whole: 4096 x 100 at 16
+    // processes 1563 -> 1371 us, 16384 x 128 1964 -> 1712, rl 4096 x 32 210.5 -> 203.6, HARQ-IR 1024 x 16 243 -> 226.
     uint32_t hmeta[P];
     int hlo[P], hrdy[P];
     const bool read_h = pm.fading && !(n_rows > 0 && (rows[0].flags & 4) && rows[0].rho == 0.0f);
@@ -2020,8 +2020,8 @@ __global__ __launch_bounds__(STEP_WAVE * (RBT > STEP_WAVE ? RBT / STEP_WAVE : 1)
                     if (cl.use_int) x = x - ((10.0f * log10f(cl.noise_mw + s_if[serv * S + s])) - ni_la[s]);
                 nan |= x != x;
                 xs[s] = x;
-                // (the mean-dB row. Not with HARQ-IR, which decodes on the log-sum: the row lies over the pair list that
-                // held_lse writes before its first barrier, with an even RBG count over another wavefront's)
+                // (the mean-dB row. Not with HARQ-IR, which decodes on the log-sum: the row lies over the pair list
+                // that held_lse writes before its first barrier, with an even RBG count over another wavefront's)
                 if constexpr (!IR) if (!pm.eesm) s_x[s * CW + lane] = x;
             }
             // the EESM log-sum of the held RBGs (lse_eesm of the linear SINR per RBG)

@@ -7,7 +7,8 @@
 // this replaces, kept a lane mask per element and per call site alive over the whole step: 1066 spilled scalar
 // registers in the Wi-Fi mean-field step at one AP, read back by lane reads in every sub-step, and 276 vector
 // registers, one wavefront per SIMD; the present step spills 164 and has 175, two wavefronts. 2048 envs of 16 robots,
-// one env per wavefront: 437 us a step before, 278 after.) A zero added to a partial sum changes no bit of it: the sums begin at +0.0, so none is -0.0.
+// one env per wavefront: 437 us a step before, 278 after.) A zero added to a partial sum changes no bit of the result:
+// the last sum begins at +0.0, so none of it is -0.0.
 #pragma once
 
 #ifdef __HIPCC__

@@ -2,7 +2,8 @@
 env, so the reference trajectories, whose batches are small, run that layout alone by default; here they run in every
 narrower one (INET_NR_LANES: several envs per wavefront, the segment's reductions and exchanges over part of it, each
 lane's own terms of several cells' interference, the 32-lane builds): teacher-forced and free running on every
-one-wavefront trajectory, with the bounds of the trajectories' own tests, and the idle and busy slots against the oracle."""
+one-wavefront trajectory, with the bounds of the trajectories' own tests, and the idle and busy slots against the
+oracle."""
 import pytest
 import torch
 

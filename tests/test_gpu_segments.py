@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 LENA = dict(pf_update="rbg", pf_avg_idle="freeze", ul_retx_sched="tdma", ul_amc_alloc="previous",
             harq_combining="ir_lena", tr38901_los="stochastic")
-# name -> config, R, envs of the large batch: more wavefronts at the next width than are resident (one cell 2048, several
-# cells 1024)
+# name -> config, R, envs of the large batch: more wavefronts at the next width than are resident (one cell 2048,
+# several cells 1024)
 CASES = {
     "plumbing R=5": (lambda: S.plumbing_config(), 5, 8200),                       # 8 lanes against 64
     "plumbing R=8, 16 lanes": (lambda: S.plumbing_config(), 8, 4100),

@@ -43,7 +43,8 @@ def width(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-std=c++17", f"-I{CSRC}", "-o", str(d / "drv"), str(d / "drv.cpp")], check=True)
 
     def run(rows):
-        """[(lanes, {width: LDS bytes of a wavefront})] of rows (E, rb0, occ, n_ul, drop, max_tx, nc, S, ir, common[, waves])."""
+        """[(lanes, {width: LDS bytes of a wavefront})] of rows (E, rb0, occ, n_ul, drop, max_tx, nc, S, ir, common[,
+        waves])."""
         text = "\n".join(" ".join(str(int(v)) for v in (tuple(r) + (1,))[:11]) for r in rows)
         out = subprocess.run([str(d / "drv")], input=text,
                              capture_output=True, text=True, check=True).stdout.split("\n")
@@ -125,7 +126,8 @@ def test_static_lds_covers_the_compiled_kernels(width):
         if m:
             S, _, ir, _, rbt, nc, fx = (int(v) for v in m.groups())
             found.setdefault((S, nc, ir, int(fx != 0), max(1, rbt // 64)), set()).add(lds)
-    assert {k[4] for k in found} == {1, 2, 4} and {k[1] for k in found} == {1, 2, 3, 4, 5, 6, 7} and {k[0] for k in found if k[1] == 1} >= {8, 13, 18}
+    assert {k[4] for k in found} == {1, 2, 4} and {k[1] for k in found} == {1, 2, 3, 4, 5, 6, 7}
+    assert {k[0] for k in found if k[1] == 1} >= {8, 13, 18}
     rows = [(1, 64, 1, 0, 0, -1, nc, S, ir, common, W) for S, nc, ir, common, W in found]
     for (k, have), (_, lds) in zip(found.items(), width(rows)):
         want = lds[64] - (8 * k[1] * k[0] if k[1] > 1 else 0)      # (less the N+I rows, dynamic)
