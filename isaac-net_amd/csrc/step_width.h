@@ -59,7 +59,8 @@ int seg_width(int E, int rb0, int occ, L lds) {
         const int64_t waves = ((int64_t)E * 2 * rb + STEP_WAVE - 1) / STEP_WAVE;
         const int64_t need = ((int64_t)lds(2 * rb) + 1279) / 1280 * 1280, held = need > 0 ? LDS / need : 0;
         const int64_t room = CUS * (held < 4 * occ ? held : 4 * occ);
-        if (waves > room) break;
+        // (a width whose envs' rows do not fit a CU, several cells with few robots per env, is passed over)
+        if (waves > room && lds(rb) + 16384 <= CU_LDS) break;
         rb *= 2;
     }
     return rb;
