@@ -91,7 +91,7 @@ def test_wavefronts_of_a_widened_batch_are_resident(width):
     ((4096, 32, 2, 10, 0, 5, 1, 13, 0, 1), 32),
     ((4096, 8, 2, 0, 0, 5, 1, 13, 0, 1), 32),         # (the downlink: no history)
     ((2048, 8, 2, 10, 0, 5, 1, 13, 0, 1), 64),
-    ((5000, 1, 1, 60, 1, 4, 7, 14, 0, 0), 2)])         # (64 envs per wavefront: their N+I rows exceed the CU)
+    ((50000, 1, 1, 60, 1, 4, 7, 14, 0, 0), 2)])         # (64 envs per wavefront: their N+I rows exceed the CU)
 def test_measured_batches(width, row, lanes):
     assert width([row])[0][0] == lanes
 
